@@ -1,7 +1,8 @@
 """Builds the package's native libraries in-tree.
 
     libgasal2_amd.so    HIP kernels (gfx950) + the host runtime of the C/C++ API
-                        (kernels.hip: the alignment pipeline; band.hip: learned band;
+                        (kernels.hip: the alignment pipeline; wave.hip: its packed
+                        one-wave path; band.hip: learned band;
                         noalloc.hip: the entry point that allocates nothing;
                         stream.cpp: FASTA/FASTQ reader and the multi-storage driver,
                         sam.cpp: CIGAR text and SAM records)
@@ -14,6 +15,7 @@ Run as ``python -m gasal2_amd.build``.  Every call recompiles.
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -42,13 +44,15 @@ def build_synth():
 
 def build_lib():
     out = os.path.join(HERE, "libgasal2_amd.so")
-    objs = []
-    for src in ("kernels.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
+    objs, cmds = [], []
+    for src in ("kernels.hip", "wave.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
         obj = os.path.join(CSRC, "_build", src + ".o")
         os.makedirs(os.path.dirname(obj), exist_ok=True)
         lang = ["-x", "hip"] if src.endswith(".hip") else []
-        _run([HIPCC] + HIP_FLAGS + lang + ["-c", os.path.join(CSRC, src), "-o", obj])
+        cmds.append([HIPCC] + HIP_FLAGS + lang + ["-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
+    with ThreadPoolExecutor(4) as pool:   # one compiler process per source
+        list(pool.map(_run, cmds))
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", out] + objs)
     return out
 

@@ -80,6 +80,12 @@ struct G2Dev {
     int32_t pk16s;                   // SEMI_GLOBAL (tails none / target) in packed 16-bit halves (semi_pass_pk)
     int32_t enc_s, enc_cb;           // position encoding: h << enc_s | ~strip << (3+enc_cb) | ~col << 3 | 7-row
     uint32_t enc_cm, enc_sm;         // column / strip field masks
+    // packed one-wave path (wave.hip): every pair on a group of lanes, the
+    // first wave_coop sorted slots on a block of four waves, the next wave64
+    // on 64 lanes, the rest on 16.  0: off, 1: cells
+    // ranked with their row (LOCAL: H <= 8191), 2: H alone.  When the census
+    // refuses the score tables the lane kernels run the batch instead.
+    uint32_t wave, wave_coop, wave64;
     // intra-pair wavefront for long pairs (LOCAL score + ends): pairs whose
     // shape passes wf_min_tw / wf_min_cells are sorted first and taken from an
     // atomic queue (aux[1], count in aux[2]) by the first wf_blocks blocks.
@@ -115,6 +121,9 @@ constexpr uint32_t G2_SHAPE_BUCKETS = 1u << 17;
 // first launch error.
 hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream, G2Timing *tm);
 
+// The DP of a batch on the packed one-wave path (d.wave, wave.hip).
+hipError_t g2_wave_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
+
 // Copies the results of a sub-batch run (pairs sub.sub_idx[k]) into the main
 // batch's result arrays and CIGAR slots.
 hipError_t g2_scatter_subset(const G2Dev &sub, const G2Dev &main, bool tb, hipStream_t stream);
@@ -124,6 +133,10 @@ hipError_t g2_scatter_subset(const G2Dev &sub, const G2Dev &main, bool tb, hipSt
 // the packed 16-bit kernels and the LOCAL position encoding.
 void g2_choose_fast(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw);
 void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t eq, uint32_t et, bool banded);
+uint32_t g2_wave_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw, int32_t fast);
+bool g2_wave_pays(const G2Opts &op, uint64_t total, uint64_t longest, uint64_t steps);
+uint64_t g2_wave_steps(uint32_t qw, uint32_t tw);
+int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total);
 G2Scores g2_scores();
 
 // Dispatch policy for LOCAL (0 auto, 1 reference-order kernel only).

@@ -13,38 +13,12 @@
 // Each lane walks its pair in the reference's order (8-row strips over the
 // target, columns left to right, rows top to bottom), so every order-dependent
 // output (end tie-breaks, second best, early exits) is the reference's.
-#include "engine.h"
+#include "device.h"
 
 #include <string.h>
 #include <type_traits>
 
 namespace {
-
-constexpr int32_t MINUS_INF = -32768;   // SHRT_MIN, src/gasal_kernels.h:35
-constexpr int WAVE = 64;
-
-enum { A_GLOBAL = 1, A_SEMI_GLOBAL = 2, A_LOCAL = 3, A_BANDED = 5, A_KSW = 6 };
-enum { S_WITHOUT_START = 0, S_WITH_START = 1, S_WITH_TB = 2 };
-enum { D_NONE = 0, D_QUERY = 1, D_TARGET = 2, D_BOTH = 3 };
-
-__device__ __forceinline__ int32_t sx16(uint32_t v) { return (int32_t)(int16_t)(uint16_t)(v & 0xFFFFu); }
-// (h & 0xFFFF) | (e << 16): one byte select (bytes 0-1 of h, then bytes 0-1 of e)
-__device__ __forceinline__ uint32_t pk16(int32_t h, int32_t e) {
-    return __builtin_amdgcn_perm((uint32_t)e, (uint32_t)h, 0x05040100u);
-}
-__device__ __forceinline__ int32_t t16(int32_t v) { return (int32_t)(int16_t)(uint16_t)((uint32_t)v & 0xFFFFu); }
-__device__ __forceinline__ int32_t dregs(uint32_t len) { return (int32_t)((len >> 3) + ((len & 7) ? 1 : 0)); }
-
-// DEV_GET_SUB_SCORE_LOCAL (src/gasal_kernels.h:40-42, :49-51)
-__device__ __forceinline__ int32_t sub_local(const G2Scores &c, int32_t nval, uint32_t r, uint32_t g) {
-    int32_t s = (r == g) ? c.match : -c.mismatch;
-    return (r == c.n_value || g == c.n_value) ? nval : s;
-}
-// DEV_GET_SUB_SCORE_GLOBAL (src/gasal_kernels.h:44-46, :53-54)
-__device__ __forceinline__ int32_t sub_global(const G2Scores &c, uint32_t r, uint32_t g) {
-    int32_t s = (r == g) ? c.match : -c.mismatch;
-    return (c.has_np && (r == c.n_value || g == c.n_value)) ? -c.np : s;
-}
 
 struct LaneCtx {
     uint32_t grp, lane, slot, pair;
@@ -63,8 +37,6 @@ struct LaneCtx {
 // tile for eight columns.  A lane's tiles: its first chunk and the strip
 // stride in query words, taken once per kernel (one region size for all
 // groups, or per-group regions).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 // A tile's eight words are 32 contiguous bytes per lane ([lane][8] within the
 // 2 KiB chunk of a wave), so a traceback lane, whose walk has left its
 // neighbours' tiles, fetches one line per tile record instead of two; the
@@ -192,10 +164,6 @@ __global__ __launch_bounds__(256) void k_pack(const uint4 *__restrict__ in, uint
 // amounts of 32 give 0, the result of PTX shl/shr the reference relies on.
 __device__ __forceinline__ uint32_t shl32(uint32_t x, uint32_t n) { return n >= 32 ? 0u : (x << n); }
 __device__ __forceinline__ uint32_t shr32(uint32_t x, uint32_t n) { return n >= 32 ? 0u : (x >> n); }
-__device__ __forceinline__ uint32_t nib_reverse(uint32_t x) {
-    x = ((x & 0x0F0F0F0Fu) << 4) | ((x >> 4) & 0x0F0F0F0Fu);
-    return __builtin_bswap32(x);
-}
 // Complement of the packed bases, all eight nibbles at once: A (1) <-> T (4)
 // toggles bits 0 and 2, C (3) <-> G (7) bit 2; every other code is kept
 // (src/kernels/pack_rc_seqs.h:56-212 maps nibble by nibble).  Bit 4k of b0..b3
@@ -317,7 +285,6 @@ __global__ __launch_bounds__(RC_WAVES * WAVE) void k_rc(G2Dev d, int32_t n_code)
 }
 
 // ------------------------------------------------------------------ sort ----
-__device__ __forceinline__ bool census_fast(uint32_t m);
 
 // Pairs are ordered by a shape bucket, largest first, so that the 64 lanes of
 // a wave share loop bounds: a counting sort over G2_SHAPE_BUCKETS keys
@@ -492,11 +459,10 @@ __global__ __launch_bounds__(256) void k_panel(G2Dev d) {
 
 // ---------------------------------------------------------------- LOCAL -----
 // gasal_local_kernel<LOCAL,S,B> (src/kernels/local_kernel_template.h:71-519).
-__device__ __forceinline__ bool census_fast(uint32_t m);
 
 template <int START, bool SECOND>
 __global__ __launch_bounds__(64) void k_local(G2Dev d, G2Scores c) {
-    if (d.fast && (d.enc_ok || d.pk2 || ((START == S_WITHOUT_START || START == S_WITH_START) && !SECOND && d.pk16)) &&
+    if (d.fast && (d.wave || d.enc_ok || d.pk2 || ((START == S_WITHOUT_START || START == S_WITH_START) && !SECOND && d.pk16)) &&
         census_fast(d.aux[0]))
         return;   // k_local_fast handles this batch
     LaneCtx x;
@@ -651,21 +617,6 @@ __global__ __launch_bounds__(64) void k_local(G2Dev d, G2Scores c) {
 //    are taken as sign bits of differences and shifted into the column word
 //    with v_alignbit (no SGPR masks); bit order per row from the top:
 //    h!=M, h!=F_in, F restarted, E restarted.  k_get_tb decodes them.
-__device__ __forceinline__ bool census_fast(uint32_t m) { return ((m & (m >> 8)) & 0xFFu) == 0u; }
-
-// GLOBAL_SEM: DEV_GET_SUB_SCORE_GLOBAL (N is an ordinary base unless N_PENALTY).
-template <bool GLOBAL_SEM = false>
-__device__ __forceinline__ uint32_t score_lut(const G2Scores &c, int32_t nval, uint32_t census, uint32_t tnib) {
-    uint32_t lut = 0;
-#pragma unroll
-    for (uint32_t cls = 0; cls < 8; cls++) {
-        const uint32_t q = ((census >> cls) & 1u) ? cls : cls + 8u;   // the nibble this class stands for
-        int32_t s = GLOBAL_SEM ? sub_global(c, q, tnib) : sub_local(c, nval, q, tnib);
-        lut |= ((uint32_t)s & 15u) << (4 * cls);
-    }
-    return lut;
-}
-
 __device__ __forceinline__ uint32_t nib_set(uint32_t w) {
     uint32_t m = 0;
 #pragma unroll
@@ -998,20 +949,6 @@ __device__ void local_reverse_start(const G2Dev &d, const G2Scores &c, const Lan
 // those of the int32 kernels.  Ends: per strip the first column
 // whose maximum beats the strip's running best, its first row; strips merged
 // in order (the reference's first strict maximum in (strip, column, row)).
-typedef short pk16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ pk16x2 as_pk(uint32_t u) { return __builtin_bit_cast(pk16x2, u); }
-__device__ __forceinline__ uint32_t as_u32(pk16x2 v) { return __builtin_bit_cast(uint32_t, v); }
-__device__ __forceinline__ pk16x2 pmax(pk16x2 a, pk16x2 b) { return __builtin_elementwise_max(a, b); }
-// a - b per half, clamped at 0 (unsigned saturation; a, b >= 0)
-__device__ __forceinline__ pk16x2 psubsat(pk16x2 a, pk16x2 b) {
-    typedef unsigned short pu16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(pk16x2, __builtin_elementwise_sub_sat(__builtin_bit_cast(pu16x2, a),
-                                                                    __builtin_bit_cast(pu16x2, b)));
-}
-// {lo16(lo), lo16(hi)} and {hi16(lo), hi16(hi)}
-__device__ __forceinline__ uint32_t pack_lo(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x05040100u); }
-__device__ __forceinline__ uint32_t pack_hi(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
-
 __device__ void lane_local_pk(const G2Dev &d, const G2Scores &c, const LaneCtx &x, uint32_t census, bool with_start) {
     const int32_t nval = c.has_np ? -c.np : 0;
     const pk16x2 gapoe2 = {(short)c.gapoe, (short)c.gapoe}, gape2 = {(short)c.gape, (short)c.gape};
@@ -1124,6 +1061,7 @@ __device__ void tb_walk(const G2Dev &d, const G2Scores &c, uint32_t slot, const 
 template <int START, bool SECOND, bool CK = false, bool WF = true>
 __global__ __launch_bounds__(64) void k_local_fast(G2Dev d, G2Scores c) {
     const uint32_t census = d.aux[0];
+    if (d.wave && census_fast(census)) return;   // the packed one-wave path has run
     // CK with tb_fused (opt-in): each lane walks its pair's traceback after its
     // DP (the walk's memory waits overlap other waves' DP); score tables of
     // the 16 target nibbles for the walk's tile recompute
@@ -1323,14 +1261,6 @@ __global__ __launch_bounds__(64) void k_local_fast(G2Dev d, G2Scores c) {
 #endif
 // 0xFFFF in each 16-bit half whose sign bit is set (v_perm sign-byte selects)
 __device__ __forceinline__ uint32_t half_sign(uint32_t v) { return __builtin_amdgcn_perm(0u, v, 0x09090808u); }
-// h * 8 + r per half in one packed multiply-add (h >= 0, r < 8 in both halves
-// of r2): left to itself the compiler turns the product into a shift and an or
-__device__ __forceinline__ pk16x2 prank(pk16x2 h, uint32_t r2) {
-    uint32_t v;
-    asm("v_pk_mad_u16 %0, %1, 8, %2 op_sel_hi:[1,0,1]" : "=v"(v) : "v"(as_u32(h)), "s"(r2));
-    return as_pk(v);
-}
-
 template <int START, bool SECOND>
 __device__ void lane2_local_pk(const G2Dev &d, const G2Scores &c, uint32_t census, uint32_t wave, uint32_t slot0,
                                const uint32_t *lut16) {
@@ -1744,7 +1674,6 @@ __global__ __launch_bounds__(64) void k_local_band(G2Dev d, G2Scores c) {
 // Used when every value fits int16 with room for the packed minus infinity
 // (NEG16 stands for MINUS_INF: it never wins a maximum against a real value
 // in that range, so the scores are those of the int32 kernel).
-constexpr int32_t NEG16 = -30000;
 __device__ void lane_global_pk(const G2Dev &d, const G2Scores &c, const LaneCtx &x, uint32_t census) {
     const int32_t gapo = c.gapo, gape = c.gape;
     const pk16x2 gapoe2 = {(short)c.gapoe, (short)c.gapoe}, gape2 = {(short)c.gape, (short)c.gape};
@@ -1984,23 +1913,6 @@ __device__ __forceinline__ void semi_column(const G2Scores &c, int32_t nval, uin
     }
     hd = pk16(h[8], e);
 }
-// Reversed copy word k of a sequence (:244-266): base 8k+b at bits 28-4b is the
-// original base len-1-(8k+b); positions past the start are nibble 0.
-// It is the nibble-reversed 8-base window of the forward sequence that starts
-// at base len-8(k+1): one funnel shift of two forward words, then a nibble
-// reverse.
-__device__ __forceinline__ uint32_t rev_word(const uint32_t *W, int32_t len, int32_t k) {
-    const int32_t st = len - 8 * (k + 1);
-    uint32_t win;
-    if (st >= 0) {
-        const int32_t w0 = st >> 3, off = st & 7;
-        win = off == 0 ? W[w0] : __builtin_amdgcn_alignbit(W[w0], W[w0 + 1], 32 - 4 * off);
-    } else {
-        win = W[0] >> (4 * (-st));   // bases before the start are nibble 0
-    }
-    return nib_reverse(win);
-}
-
 // One pass of k_semi (forward, or with REV the WITH_START pass over reversed
 // copies) with two strips per lane in packed 16-bit halves, skewed by one
 // column as in lane_local_pk; tails that end on the target only (TT) or none.
@@ -3006,7 +2918,12 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             else k_local_band<false, false><<<grid, blk, 0, s>>>(d, sc);
             break;
         case A_LOCAL:
-            if (d.fast && d.pk2) {   // two pairs per lane: half the lane-path blocks
+            if (d.wave) {
+                const hipError_t e = g2_wave_run(sc, op, d, s);
+                if (e != hipSuccess) return e;
+                // a batch without score tables keeps one wave per long pair
+                if (d.wf_blocks) k_local_fast<S_WITHOUT_START, false><<<dim3(groups + d.wf_blocks), blk, 0, s>>>(d, sc);
+            } else if (d.fast && d.pk2) {   // two pairs per lane: half the lane-path blocks
                 const dim3 g2((groups + 1) / 2), g2w((groups + 1) / 2 + d.wf_blocks);
                 if (op.start == S_WITH_TB) {
                     if (second) k_local_pk2<S_WITH_TB, true, false><<<g2, blk, 0, s>>>(d, sc);
@@ -3050,7 +2967,10 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             }
             break;
         case A_GLOBAL:
-            if (d.fast) {
+            if (d.wave) {
+                const hipError_t e = g2_wave_run(sc, op, d, s);
+                if (e != hipSuccess) return e;
+            } else if (d.fast) {
                 if (tb) k_global<true, true><<<grid, blk, 0, s>>>(d, sc);
                 else k_global<false, true><<<grid, blk, 0, s>>>(d, sc);
             }
@@ -3058,15 +2978,19 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             else k_global<false, false><<<grid, blk, 0, s>>>(d, sc);
             break;
         case A_SEMI_GLOBAL:
+            if (d.wave) {
+                const hipError_t e = g2_wave_run(sc, op, d, s);
+                if (e != hipSuccess) return e;
+            }
             if (op.start == S_WITH_START) {
-                if (d.fast) {
+                if (d.fast && !d.wave) {
                     if (second) launch_semi_ht<S_WITH_START, true, true>(op.head, op.tail, grid, blk, s, d, sc);
                     else launch_semi_ht<S_WITH_START, false, true>(op.head, op.tail, grid, blk, s, d, sc);
                 }
                 if (second) launch_semi_ht<S_WITH_START, true, false>(op.head, op.tail, grid, blk, s, d, sc);
                 else launch_semi_ht<S_WITH_START, false, false>(op.head, op.tail, grid, blk, s, d, sc);
             } else {
-                if (d.fast) {
+                if (d.fast && !d.wave) {
                     if (second) launch_semi_ht<S_WITHOUT_START, true, true>(op.head, op.tail, grid, blk, s, d, sc);
                     else launch_semi_ht<S_WITHOUT_START, false, true>(op.head, op.tail, grid, blk, s, d, sc);
                 }

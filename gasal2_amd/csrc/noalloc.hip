@@ -183,6 +183,17 @@ extern "C" int32_t gasal2_aln_noalloc(const void *query_batch, const void *targe
     const G2Scores sc = g2_scores();
     g2_choose_fast(d, op, sc, qw, tw);
     g2_choose_packed(d, op, sc, qw, tw, false);
+    // only the declared maxima are known here: every pair counts as the longest
+    const uint64_t cells = 64ull * qw * tw, total = cells * n;
+    d.wave = g2_wave_fits(op, sc, qw, tw, d.fast);
+    if (d.wave && (g2_get_dispatch() == 3 ||
+                   (g2_get_dispatch() == 0 && g2_wave_pays(op, total, cells, g2_wave_steps(qw, tw) * n)))) {
+        const int lanes = g2_wave_lanes(qw, tw, total);
+        d.wave_coop = lanes == 256 ? n : 0;
+        d.wave64 = lanes == 64 ? n : 0;
+    } else {
+        d.wave = 0;
+    }
 
     const uint32_t nb = (n + 255) / 256;
     k_noalloc_zero<<<1, 64, 0, stream>>>(aux + AUX_BAD, 1);   // rejected-pair counter

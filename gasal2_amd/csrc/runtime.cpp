@@ -17,6 +17,7 @@
 #include <atomic>
 #include <mutex>
 #include <algorithm>
+#include <cmath>
 
 // ------------------------------------------------------------ globals ------
 // An order chain (the batch order below).
@@ -968,6 +969,75 @@ extern "C" void gasal_gpu_mem_free(gasal_gpu_storage_t *gpu_storage, Parameters 
 // Packed and table kernels for a batch: the choices depend only on the
 // mode, the scores and the largest shape the lane path runs (eq query words,
 // et target words); shared by the storage path and gasal2_aln_noalloc.
+// Whether the packed one-wave path (wave.hip) can run a batch whose largest
+// pair has qw query and tw target words: its G2Dev::wave value, 0 when a value
+// could leave 16 bits.  LOCAL holds E and F at or above 0, so only H <= the
+// best substitution score times the shorter side counts; ranked cells need
+// H <= 8191.  GLOBAL and SEMI_GLOBAL: H is at least the all-gap alignment's
+// score -- one open along each side, an extension per row and column (a SEMI
+// reverse run may start above the target: at most qw + 2 strips more) -- and E
+// and F are an open below an H; all must stay above NEG16 and its extension.
+uint32_t g2_wave_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw, int32_t fast) {
+    if (!fast || !g_pk16_mode || op.second || op.start == WITH_TB || op.banded) return 0;
+    if (op.algo != LOCAL && op.algo != GLOBAL && op.algo != SEMI_GLOBAL) return 0;
+    if (sc.gapo < 0 || sc.gape < 0 || sc.gapo > 16000 || sc.gape > 255) return 0;
+    if (8ull * qw + 256 > 65535) return 0;   // steps of a pass are held in 16 bits
+    const int64_t nval = sc.has_np ? -sc.np : 0;
+    const int64_t up = std::max<int64_t>({sc.match, -(int64_t)sc.mismatch, nval, 0});
+    const int64_t down = std::max<int64_t>({-(int64_t)sc.match, sc.mismatch, -nval, 0});
+    const int64_t hmax = up * 8 * std::min<int64_t>(qw, tw);
+    if (op.algo == LOCAL) return hmax <= 8191 ? 1 : (hmax <= 32000 ? 2 : 0);
+    const int64_t low = 3ll * sc.gapoe + sc.gape * (16ll * std::max(qw, tw) + 64) + 2 * down;
+    return hmax <= 32000 && low <= 29000 ? 1 : 0;
+}
+
+// Whether that path beats the lane kernels on a batch.  total and longest:
+// padded cells of the batch and of the longest pair the lane kernels would run;
+// steps: the path's lane-steps on 16 lanes, g2_wave_steps() of every pair.
+// The lane kernels are bound by the longer of the longest pair's serial time
+// and their rate, with part of the shorter one on top; this path by its rate.
+// Constants: 1,000 to 300,000 pairs of 150 x 250 and of 100-300 x 100-400 bases
+// on one MI355X, e.g. LOCAL on the first, this path / lanes: 10,000 pairs
+// 0.33 / 1.07 ms, 100,000 1.56 / 1.74, 300,000 4.0 / 3.6; on the second
+// 100,000 pairs 2.9 / 3.3, 300,000 8.2 / 5.7.
+bool g2_wave_pays(const G2Opts &op, uint64_t total, uint64_t longest, uint64_t steps) {
+    struct Rates { double lane_serial, lane, wave; };   // seconds a cell; cells a second; lane-steps' cells a second
+    const Rates local = {24e-9, 3.2e12, 3.45e12}, local_start = {40e-9, 1.75e12, 2.1e12}, global = {15e-9, 4.1e12, 4.6e12},
+                semi = {16e-9, 4.7e12, 4.4e12}, semi_start = {32e-9, 2.4e12, 2.2e12};
+    const bool start = op.start == WITH_START;
+    const Rates &r = op.algo == LOCAL ? (start ? local_start : local) : (op.algo == GLOBAL ? global : (start ? semi_start : semi));
+    const double serial = r.lane_serial * (double)longest, rate = (double)total / r.lane;
+    return (double)steps / r.wave < std::max(serial, rate) + 0.2 * std::min(serial, rate);
+}
+
+// Cells' worth of lane-steps of a pair on 16 lanes: passes of 256 rows, each
+// its columns and 32 steps to fill.
+uint64_t g2_wave_steps(uint32_t qw, uint32_t tw) { return 2048ull * ((tw + 31) / 32) * (qw + 4); }
+
+// Lanes of that path for a pair: 256 (a block's four waves) or 64 when the pair
+// would otherwise outlast its share of a batch of `total` cells, 64 also where
+// the share of lanes and steps that hold cells is close to that of 16 lanes.
+// Measured on 20,000 pairs of 50-5000 bases, LOCAL: without the 256 10.5 ms,
+// with it 4.1; on 100,000 pairs 14.4 and 14.1.
+int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total) {
+    // least query words for which 64 lanes hold at least 0.85 of the share of 16
+    static const std::vector<uint32_t> wide = [] {
+        std::vector<uint32_t> v(1024);
+        for (uint32_t t = 0; t < 1024; t++) {
+            const double full = ((t + 31) / 32) * 16.0 / (((t + 127) / 128) * 64.0) / 0.85;   // of 16 lanes to 64
+            uint32_t q = 0;
+            while (q < 1024 && (8 * q + 32) * full < 8 * q + 128) q++;
+            v[t] = q;
+        }
+        return v;
+    }();
+    if (tw <= 32) return 16;
+    const double cells = 64.0 * qw * tw;
+    if (tw > 128 && cells > 2.3e-4 * (double)total) return 256;
+    if (cells > 4e-4 * (double)total) return 64;
+    return qw >= wide[std::min<uint32_t>(tw, 1023)] ? 64 : 16;
+}
+
 void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t eq, uint32_t et, bool banded) {
     auto bl = [](uint64_t v) { int b = 0; while (v) { b++; v >>= 1; } return b; };
     // Packed 16-bit LOCAL (score and ends; WITH_START then runs the int32
@@ -1385,6 +1455,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // census to allow the score tables; the host count only sizes the launch.
     uint32_t eq = qw, et = tw;   // largest shape the one-lane-per-pair kernels see
     uint32_t nlong = 0;
+    bool switched = g_wf_user;   // lane / one-wave thresholds set by the caller or the tuner
     if (d.fast && op.algo == LOCAL && (op.start == WITHOUT_START || (op.start == WITH_TB && !px.banded)) && !op.second &&
         g2_get_dispatch() != 2) {
         uint32_t min_tw = g_wf_min_tw, min_cells = g_wf_min_cells, max_blocks = g_wf_max_blocks;
@@ -1403,6 +1474,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                     break;
                 }
         }
+        switched |= tuned;
         // the small-batch rule yields to user and tuned thresholds
         const bool few = g2_get_dispatch() == 0 && !g_wf_user && !tuned &&
                          (uint64_t)n <= (uint64_t)g2_cu_count() * (op.start == WITH_TB ? WF_FEW_PER_CU_TB : WF_FEW_PER_CU);
@@ -1557,6 +1629,29 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         s->packed_tb_matrix_size = m->tb_bytes / 16;
     }
     g2_choose_packed(d, op, sc, eq, et, px.banded);
+    if (!px.banded) d.wave = g2_wave_fits(op, sc, qw, tw, d.fast);
+    if (d.wave) {
+        // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
+        const bool mixed = op.algo == LOCAL && op.start == WITHOUT_START;
+        uint64_t total = 0, longest = 0, steps = 0;
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
+            const uint64_t cells = 64ull * kq * kt;
+            total += cells;
+            steps += g2_wave_steps(kq, kt);
+            if (!mixed || kt < g_wf_min_tw || cells < g_wf_min_cells) longest = std::max(longest, cells);
+        }
+        const int policy = g2_get_dispatch();
+        if (policy == 3 || (policy == 0 && !(mixed && switched) && g2_wave_pays(op, total, longest, steps))) {
+            for (uint32_t k = 0; k < n && tw > 32; k++) {
+                const int lanes = g2_wave_lanes(g2_regs(hq[k]), g2_regs(ht[k]), total);
+                d.wave_coop += lanes == 256;
+                d.wave64 += lanes == 64;
+            }
+        } else {
+            d.wave = 0;
+        }
+    }
 }
 
 G2Scores scores_now() { return g_scores; }
@@ -1589,7 +1684,7 @@ void upload_async(gasal_gpu_storage_t *s, uint32_t n, Parameters *params) {
 // trigger a new capture.  The program holds kernels only (no memset or copy
 // nodes).  Timed runs (per-stage events) launch eagerly.
 hipError_t launch_program(Impl *m, const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t st) {
-    m->last_paths = ((d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16) ? 1 : 0) | (d.wf_blocks ? 2 : 0) | (d.tbh ? 4 : 0);
+    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh ? 4 : 0);
     if (!g_graph_mode || m->tm.enabled) return g2_run(sc, op, d, st, &m->tm);
     const bool same = m->g_valid && memcmp(&m->g_dev, &d, sizeof(d)) == 0 && memcmp(&m->g_sc, &sc, sizeof(sc)) == 0 &&
                       memcmp(&m->g_op, &op, sizeof(op)) == 0;
