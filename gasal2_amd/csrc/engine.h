@@ -46,7 +46,7 @@ struct G2Dev {
     uint8_t *cigar_qlayout;          // reference layout: CIGAR at query offsets
     // workspace
     uint32_t *keys, *perm;           // shape key and sorted permutation, n each
-    uint32_t *hist;                  // G2_SHAPE_BUCKETS counters / bucket offsets
+    uint32_t *hist;                  // G2_SHAPE_BUCKETS counters / bucket offsets, then G2_SHAPE_ROWS row sums
     uint32_t *bnd;                   // boundary rows: per group bnd_cols*64 dwords
     uint32_t bnd_cols;
     uint32_t *tb;                    // direction words (or tile left states): per group tb_tw*tb_qw8*64
@@ -116,6 +116,7 @@ struct G2Timing {
 
 // Shape buckets of the pair ordering (long flag, 8-bit query and target word classes).
 constexpr uint32_t G2_SHAPE_BUCKETS = 1u << 17;
+constexpr uint32_t G2_SHAPE_ROWS = G2_SHAPE_BUCKETS / 256;   // one long flag and query class each
 
 // Enqueue the whole device pipeline on `stream`.  Returns hipSuccess or the
 // first launch error.

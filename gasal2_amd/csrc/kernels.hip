@@ -347,40 +347,52 @@ __global__ __launch_bounds__(KH_THREADS) void k_keys(G2Dev d) {
         const uint32_t key = pair_key(d, k, lng);
         d.keys[k] = key;
         const int h = kh_slot(tkey, key);
-        if (h >= 0) atomicAdd(&tcnt[h], 1u);
-        else atomicAdd(&d.hist[key], 1u);
+        if (h >= 0) {
+            atomicAdd(&tcnt[h], 1u);
+        } else {
+            atomicAdd(&d.hist[key], 1u);
+            atomicAdd(&d.hist[G2_SHAPE_BUCKETS + (key >> 8)], 1u);
+        }
         if (lng) atomicAdd(&nlong, 1u);
     }
     __syncthreads();
     for (uint32_t i = t; i < KH_SLOTS; i += KH_THREADS)
-        if (tcnt[i]) atomicAdd(&d.hist[tkey[i]], tcnt[i]);
+        if (tcnt[i]) {
+            atomicAdd(&d.hist[tkey[i]], tcnt[i]);
+            atomicAdd(&d.hist[G2_SHAPE_BUCKETS + (tkey[i] >> 8)], tcnt[i]);
+        }
     if (t == 0 && nlong) atomicAdd(&d.aux[2], nlong);
 }
 
 // Exclusive scan of the histogram in descending key order, in place: hist[b]
-// becomes the first sorted slot of bucket b.  One block of 1024 threads, each
-// owning G2_SHAPE_BUCKETS / 1024 consecutive buckets.
-__global__ __launch_bounds__(1024) void k_scan_desc(uint32_t *hist) {
-    constexpr uint32_t PER = G2_SHAPE_BUCKETS / 1024;
-    __shared__ uint32_t part[1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t hi = G2_SHAPE_BUCKETS - 1 - t * PER;   // this thread's buckets: hi, hi-1, ..., hi-PER+1
-    uint32_t sum = 0;
-    for (uint32_t i = 0; i < PER; i++) sum += hist[hi - i];
-    part[t] = sum;
+// becomes the first sorted slot of bucket b.  One block per row of 256 buckets
+// (one long flag and query class): the row's first slot is the sum of the
+// row sums above it (the last G2_SHAPE_ROWS entries of hist, counted by
+// k_keys), then a scan of its own buckets; rows with no pair are left at 0.
+// Bound by two dependent round trips to L2.  One block scanning all buckets
+// took 53 us whatever the batch, each thread reading 128 counters one after
+// the other.
+__global__ __launch_bounds__(256) void k_scan_desc(uint32_t *hist) {
+    __shared__ uint32_t part[4], base[4];
+    const uint32_t t = threadIdx.x, lane = t & (WAVE - 1), wv = t / WAVE, row = blockIdx.x;
+    const uint32_t *rows = hist + G2_SHAPE_BUCKETS;
+    if (rows[row] == 0) return;   // the whole block
+    uint32_t above = 0;
+    for (uint32_t r = t; r < G2_SHAPE_ROWS; r += 256) above += r > row ? rows[r] : 0u;
+    const uint32_t v = hist[row * 256 + 255 - t];   // descending order
+    uint32_t inc = v;
+#pragma unroll
+    for (uint32_t off = 1; off < WAVE; off <<= 1) {
+        const uint32_t o = __shfl_up(inc, off);
+        inc += lane >= off ? o : 0u;
+    }
+#pragma unroll
+    for (uint32_t off = 32; off > 0; off >>= 1) above += __shfl_xor(above, off);
+    if (lane == WAVE - 1) { part[wv] = inc; base[wv] = above; }
     __syncthreads();
-    for (uint32_t off = 1; off < 1024; off <<= 1) {   // Hillis-Steele inclusive scan
-        const uint32_t v = t >= off ? part[t - off] : 0u;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    uint32_t run = part[t] - sum;
-    for (uint32_t i = 0; i < PER; i++) {
-        const uint32_t c = hist[hi - i];
-        hist[hi - i] = run;
-        run += c;
-    }
+    uint32_t first = base[0] + base[1] + base[2] + base[3] + inc - v;
+    for (uint32_t w = 0; w < wv; w++) first += part[w];
+    hist[row * 256 + 255 - t] = first;
 }
 
 // Places each pair at its bucket's next free slot.  As in k_keys, a block
@@ -649,14 +661,25 @@ __global__ __launch_bounds__(256) void k_census(const uint32_t *__restrict__ pq,
     }
     if (gtid < (nq & 3u)) m |= nib_set(pq[(nq & ~3u) + gtid]);
     if (gtid < (nt & 3u)) m |= nib_set(pt[(nt & ~3u) + gtid]);
-    // wave reduction then one atomic per wave
+    // One value per block, and an atomic only when it adds a bit: a batch
+    // holds about five nibbles, so nearly every block finds its bits set.  (An
+    // atomic per wave on this one word serialised: 100 us on 2048 blocks.)
+    __shared__ uint32_t part[4];
     for (int off = 32; off > 0; off >>= 1) m |= __shfl_xor(m, off);
-    if ((threadIdx.x & 63) == 0 && m) atomicOr(out, m);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x / 64] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = part[0] | part[1] | part[2] | part[3];
+        if (m & ~__hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(out, m);
+    }
 }
 
-__global__ void k_zero_u32(uint32_t *p, uint32_t n) {
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) p[k] = 0;
+// Clears the batch's counters: the first four words of aux and the histogram.
+__global__ __launch_bounds__(256) void k_zero_counters(uint32_t *aux, uint32_t *hist) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < 4) aux[k] = 0;
+    for (uint32_t i = k; i < (G2_SHAPE_BUCKETS + G2_SHAPE_ROWS) / 4; i += gridDim.x * blockDim.x)
+        reinterpret_cast<uint4 *>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 // ------------------------------------------------ LOCAL, one wave per pair ----
@@ -2888,7 +2911,7 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
     if (timing) (void)hipEventRecord(tm->ev[2], s);
     // aux[0] nibble census over the packed batch for the score-table kernels;
     // aux[1..2] long-pair queue head and count
-    k_zero_u32<<<1, 64, 0, s>>>(d.aux, 4);
+    k_zero_counters<<<128, 256, 0, s>>>(d.aux, d.hist);
     if (d.fast) {
         // packed words of the batch: the byte counts count bases (8 per word) with or without isPacked
         const uint32_t qw = d.q_bytes / 8;
@@ -2899,10 +2922,9 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
     G2_LAUNCH_CHECK();
     // 3. order pairs by shape (largest first) so a wave's lanes share loop bounds;
     // long pairs for the one-wave-per-pair path sort ahead of all others
-    k_zero_u32<<<G2_SHAPE_BUCKETS / 256, 256, 0, s>>>(d.hist, G2_SHAPE_BUCKETS);
     const uint32_t nkh = (d.n + KH_CHUNK - 1) / KH_CHUNK;
     k_keys<<<nkh, KH_THREADS, 0, s>>>(d);
-    k_scan_desc<<<1, 1024, 0, s>>>(d.hist);
+    k_scan_desc<<<G2_SHAPE_ROWS, 256, 0, s>>>(d.hist);
     k_scatter<<<nkh, KH_THREADS, 0, s>>>(d);
     if (d.qpan) k_panel<<<(d.n + WAVE - 1) / WAVE, 256, 0, s>>>(d);
     G2_LAUNCH_CHECK();

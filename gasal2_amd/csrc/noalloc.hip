@@ -15,8 +15,11 @@ namespace {
 // histogram, boundary rows and the outputs the caller does not ask for.
 // Each device holds its own copy until the process ends; calls that overlap
 // on one device race on it.
+// What a batch may need of its own is NOALLOC_SCRATCH_BYTES; the histogram's
+// row sums, the same for every batch, lie beside it.
 constexpr size_t NOALLOC_SCRATCH_BYTES = 32u << 20;
-static __device__ __align__(256) uint8_t scratch[NOALLOC_SCRATCH_BYTES];
+constexpr size_t NOALLOC_FIXED_BYTES = (size_t)G2_SHAPE_ROWS * 4;
+static __device__ __align__(256) uint8_t scratch[NOALLOC_SCRATCH_BYTES + NOALLOC_FIXED_BYTES];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
@@ -123,12 +126,13 @@ extern "C" int32_t gasal2_aln_noalloc(const void *query_batch, const void *targe
     const size_t o_qlen = take((size_t)n * 4), o_tlen = take((size_t)n * 4);
     const size_t o_qop = take(n), o_top = take(n);
     const size_t o_keys = take((size_t)n * 4), o_perm = take((size_t)n * 4);
-    const size_t o_hist = take((size_t)G2_SHAPE_BUCKETS * 4);
+    const size_t o_hist = take((size_t)(G2_SHAPE_BUCKETS + G2_SHAPE_ROWS) * 4);
     const size_t o_aux = take(256 + 4096);
     const size_t o_bnd = take((size_t)groups * bnd_cols * 64 * 4);
     const size_t o_dummy = take((size_t)n * 4 * 5);
-    if (off > NOALLOC_SCRATCH_BYTES)
-        return fail("[GASAL ERROR:] gasal2_aln_noalloc: the batch needs %zu bytes of scratch, more than %zu\n", off,
+    if (off > NOALLOC_SCRATCH_BYTES + NOALLOC_FIXED_BYTES)
+        return fail("[GASAL ERROR:] gasal2_aln_noalloc: the batch needs %zu bytes of scratch, more than %zu\n",
+                    off - NOALLOC_FIXED_BYTES,
                     (size_t)NOALLOC_SCRATCH_BYTES);
 
     G2Dev d;

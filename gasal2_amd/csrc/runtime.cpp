@@ -1383,7 +1383,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         }
         m->n_cap = n;
     }
-    if (!m->hist) G2_CHECK(hipMalloc((void **)&m->hist, (size_t)G2_SHAPE_BUCKETS * 4));
+    if (!m->hist) G2_CHECK(hipMalloc((void **)&m->hist, (size_t)(G2_SHAPE_BUCKETS + G2_SHAPE_ROWS) * 4));
     const uint32_t bnd_cols = 8 * qw + 8;
     ensure(m->bnd, m->bnd_bytes, (size_t)groups * bnd_cols * 64 * 4);
     const bool tb_on = op.start == WITH_TB;
