@@ -2,7 +2,7 @@
 
     libgasal2_amd.so    HIP kernels (gfx950) + the host runtime of the C/C++ API
                         (kernels.hip: the alignment pipeline; wave.hip: its packed
-                        one-wave path; band.hip: learned band;
+                        one-wave path; ksw.hip: KSW in packed strips; band.hip: learned band;
                         noalloc.hip: the entry point that allocates nothing;
                         stream.cpp: FASTA/FASTQ reader and the multi-storage driver,
                         sam.cpp: CIGAR text and SAM records)
@@ -45,7 +45,7 @@ def build_synth():
 def build_lib():
     out = os.path.join(HERE, "libgasal2_amd.so")
     objs, cmds = [], []
-    for src in ("kernels.hip", "wave.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
+    for src in ("kernels.hip", "wave.hip", "ksw.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
         obj = os.path.join(CSRC, "_build", src + ".o")
         os.makedirs(os.path.dirname(obj), exist_ok=True)
         lang = ["-x", "hip"] if src.endswith(".hip") else []

@@ -67,6 +67,7 @@ struct G2Dev {
     int32_t *eh;                     // KSW rows: per group eh_cols*64*2 ints
     uint32_t eh_cols;
     int32_t ksw16;                   // KSW rows as packed uint16 (H, E): values fit 16 bits
+    uint32_t ksw_pk;                 // KSW in packed strips (ksw.hip); k_ksw runs the pairs it lists in keys (aux[3])
     uint32_t *aux;                   // small device counters (work queue etc.)
     uint32_t *sink;                  // 4 KiB a kernel may write discarded records to (never read)
     // score-table kernels (k_local_fast, k_global / k_semi LUT variants): 0 =
@@ -124,6 +125,9 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
 
 // The DP of a batch on the packed one-wave path (d.wave, wave.hip).
 hipError_t g2_wave_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
+
+// KSW in packed 16-bit strips (d.ksw_pk, ksw.hip).
+hipError_t g2_ksw_packed(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
 
 // Copies the results of a sub-batch run (pairs sub.sub_idx[k]) into the main
 // batch's result arrays and CIGAR slots.

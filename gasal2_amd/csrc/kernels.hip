@@ -2315,6 +2315,10 @@ __global__ __launch_bounds__(64) void k_ksw(G2Dev d, G2Scores c, int32_t w, int3
                                             uint32_t qlds) {
     const uint32_t census = d.aux[0];
     if (LUT != (d.fast && census_fast(census))) return;
+    if (LUT && d.ksw_pk) {   // only the pairs the packed kernel listed
+        if (blockIdx.x * WAVE + threadIdx.x >= d.aux[3]) return;
+        d.perm = d.keys;
+    }
     LaneCtx x;
     if (!lane_setup(d, x)) return;
     if (QL)
@@ -3031,6 +3035,10 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             const uint32_t qw = (d.eh_cols - 2 + 7) / 8;
             const uint32_t qlds = qw <= 128 ? qw : 0;
             const size_t lds = (size_t)qlds * WAVE * 4;
+            if (d.ksw_pk) {
+                const hipError_t e = g2_ksw_packed(sc, op, d, s);
+                if (e != hipSuccess) return e;
+            }
             if (d.ksw16) {
                 if (qlds) {
                     k_ksw<true, true, true><<<grid, blk, lds, s>>>(d, sc, op.ksw_w, op.ksw_zdrop, op.ksw_eb, qlds);

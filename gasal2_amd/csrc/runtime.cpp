@@ -1437,12 +1437,14 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     d.tb = m->tb; d.tb_tw = tw; d.tb_qw8 = 8 * qw;
     d.eh = m->eh; d.eh_cols = eh_cols;
     d.ksw16 = 0;
+    uint64_t ksw_hmax = ~0ull;
     if (op.algo == KSW && s->host_seed_scores && !px.sub) {   // every KSW value lies in [0, h0 + match * min(Lq, Lt)]
         uint64_t hmax = 0;
         for (uint32_t k = 0; k < n; k++)
             hmax = std::max<uint64_t>(hmax, (uint64_t)s->host_seed_scores[k] +
                                                 (uint64_t)std::max(g_scores.match, 0) * std::min(hq[k], ht[k]));
         if (hmax <= 65535 && g_pk16_mode) d.ksw16 = 1;
+        ksw_hmax = hmax;
     }
     if (!m->aux) G2_CHECK(hipMalloc((void **)&m->aux, 256 + 4096));
     d.aux = m->aux;
@@ -1532,9 +1534,15 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             }
         }
     }
-    // Transposed sequence panels for the fast LOCAL lane path (k_panel): groups
-    // after the long pairs, eq query words and et target words each.
-    if (g_panels && d.fast && op.algo == LOCAL && !px.banded && n > nlong) {
+    // KSW in packed strips: the reference's form (no band, no z-drop), ranked
+    // cells (H <= 4095), an end bonus that a gap open covers (ksw.hip).
+    if (op.algo == KSW && d.fast && g_pk16_mode && op.ksw_w < 0 && op.ksw_zdrop <= 0 && ksw_hmax <= 4095 && sc.gapo >= 0 &&
+        sc.gape >= 0 && sc.gape <= 255 && sc.gapoe >= 1 && sc.gapoe <= 16000 && op.ksw_eb <= sc.gapoe &&
+        8ull * qw + 8 <= 65535)
+        d.ksw_pk = 1;
+    // Transposed sequence panels for the fast LOCAL and KSW lane path (k_panel):
+    // groups after the long pairs, eq query words and et target words each.
+    if (g_panels && (d.ksw_pk || (d.fast && op.algo == LOCAL)) && !px.banded && n > nlong) {
         const uint64_t lgroups = ((uint64_t)(n - nlong) + 63) / 64;
         ensure(m->qpan, m->qpan_bytes, (size_t)(lgroups * eq * 256) + 256);
         ensure(m->tpan, m->tpan_bytes, (size_t)(lgroups * et * 256) + 256);
