@@ -75,6 +75,36 @@ __device__ __forceinline__ pk16x2 prank(pk16x2 h, uint32_t r2) {
     return as_pk(v);
 }
 
+// the previous lane's v within the group; the group's first lane: first
+template <int GW>
+__device__ __forceinline__ uint32_t from_above(uint32_t first, uint32_t v) {
+    static_assert(GW == 4 || GW == 16 || GW == 64, "lanes of a group");
+    const uint32_t w = (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, GW == 64 ? 0x138 : 0x111, 0xF, 0xF, false);
+    return GW == 4 && (threadIdx.x & 3u) == 0 ? first : w;
+}
+// maximum over the wave of a value that is uniform within groups of GW lanes
+template <int GW = 16>
+__device__ __forceinline__ int32_t wave_max(int32_t v) {
+#pragma unroll
+    for (int off = GW; off < WAVE; off <<= 1) v = max(v, __shfl_xor(v, off));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ pk16x2 pmaxu(pk16x2 a, pk16x2 b) {
+    typedef unsigned short pu16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(pk16x2, __builtin_elementwise_max(__builtin_bit_cast(pu16x2, a), __builtin_bit_cast(pu16x2, b)));
+}
+// 0xFFFF in each half that is not 0 (written out: the compiler makes compares
+// and selects per half of it)
+__device__ __forceinline__ uint32_t nonzero_mask(pk16x2 v) {
+    uint32_t one, m;
+    asm("v_pk_min_u16 %0, %1, 1 op_sel_hi:[1,0]" : "=v"(one) : "v"(as_u32(v)));
+    asm("v_pk_sub_i16 %0, 0, %1" : "=v"(m) : "v"(one));
+    return m;
+}
+__device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
+__device__ __forceinline__ pk16x2 set_lo(pk16x2 v, int32_t x) { return as_pk(bits_of(0xFFFFu, (uint32_t)x, as_u32(v))); }
+__device__ __forceinline__ pk16x2 set_hi(pk16x2 v, int32_t x) { return as_pk(pack_lo(as_u32(v), (uint32_t)x)); }
+
 // Stands for MINUS_INF in packed 16-bit halves: it never wins a maximum against
 // a real value of the pairs those kernels take.
 constexpr int32_t NEG16 = -30000;
@@ -95,6 +125,68 @@ __device__ __forceinline__ uint32_t rev_word(const uint32_t *W, int32_t len, int
         win = W[0] >> (4 * (-st));   // bases before the start are nibble 0
     }
     return nib_reverse(win);
+}
+
+// Recomputes one 8x8 tile's direction words (k_local_fast's sign-bit format)
+// from the checkpoints k_local_fast<.., CK> stored: the previous strip's
+// bottom row above the tile and the tile's left column state.  Same
+// recurrences and score tables (lut: the strip's eight rows, as k_local_fast
+// builds them), so the same words.
+// top: the row above, entry kk = (H at column kk - 1, E at column kk), so the
+// entry left of the tile's first column (the corner) comes with it; zero above
+// strip 0.  left: the left column state; lut: the strip's score tables (the
+// kernels store checkpoints only when the batch's nibble census allows tables).
+// The words hold the reference's nibbles (src/kernels/local_kernel_template.h
+// :45-60): [3] F continues (t <= f - extend), [2] E continues, [1:0] source:
+// diagonal 0 / 1 by the score's sign, F 3, E 2, ties in that order.
+template <bool LOCALT>
+__device__ __forceinline__ void ck_tile(const uint32_t *top, const uint32_t *left, uint32_t qword,
+                                        const uint32_t *lut, const G2Scores &c, uint32_t *ch) {
+    int32_t h[9], f[9];
+#pragma unroll
+    for (int m = 1; m < 9; m++) { h[m] = sx16(left[m - 1]); f[m] = (int32_t)left[m - 1] >> 16; }
+    const int32_t gapoe = c.gapoe, gape = c.gape;
+#pragma unroll
+    for (int kk = 0; kk < 8; kk++) {
+        const uint32_t qsh = kk < 7 ? (qword >> (26 - 4 * kk)) & 0x1Cu : (qword << 2) & 0x1Cu;
+        int32_t e = (int32_t)top[kk] >> 16;
+        int32_t p = sx16(top[kk]);
+        uint32_t dir = 0;
+#pragma unroll
+        for (int m = 1; m < 9; m++) {
+            const int32_t sc = __builtin_amdgcn_sbfe(lut[m - 1], qsh, 4);
+            const int32_t tmp = p + sc;
+            const int32_t hm = LOCALT ? max(max(max(tmp, f[m]), e), 0) : max(max(tmp, f[m]), e);
+            const int32_t t = tmp - gapoe;
+            const int32_t fx = f[m] - gape, ex = e - gape;
+            const uint32_t na = (uint32_t)(tmp - hm);                       // sign: not from the diagonal
+            dir = __builtin_amdgcn_alignbit(dir, (uint32_t)t + ~(uint32_t)fx, 31);   // sign: fx >= t
+            dir = __builtin_amdgcn_alignbit(dir, (uint32_t)t + ~(uint32_t)ex, 31);   // sign: ex >= t
+            dir = __builtin_amdgcn_alignbit(dir, na, 31);
+            // low bit: from F (hm <= f) when not diagonal, else the mismatch flag (score < 0)
+            dir = __builtin_amdgcn_alignbit(dir, (na & ((uint32_t)hm + ~(uint32_t)f[m])) | (~na & (uint32_t)sc), 31);
+            f[m] = max(t, fx);
+            e = max(t, ex);
+            p = h[m];
+            h[m] = hm;
+        }
+        ch[kk] = dir;
+    }
+}
+
+// Checkpoints of the one-wave traceback path (wavetb.hip).  A wave's region
+// is a log of its iterations: 8 KiB each, four streams of one 32-byte record a
+// lane -- left column state of the low and the high strip, bottom row of the
+// low and the high strip -- so that every store of a wave covers whole lines.
+// at: the pair's first iteration, first lane | log2(lanes of its group) << 8.
+constexpr uint32_t WV_STREAM = WAVE * 8, WV_ITER = 4 * WV_STREAM;   // dwords
+enum { WV_LEFT = 0, WV_BOTTOM = 2 };
+// iterations from a group's pass to its next one: its words, or the lanes' lag
+__device__ __forceinline__ int32_t wv_period(int32_t QW, int32_t gw) { return max(QW, gw + 1); }
+__device__ __forceinline__ uint32_t *wv_tile(const G2Dev &d, uint2 at, int32_t QW, int32_t strip, int32_t word, int32_t what) {
+    const int32_t lg = (int32_t)(at.y >> 8), gw = 1 << lg, u = strip >> 1, l = u & (gw - 1);
+    const uint32_t it = at.x + (uint32_t)((u >> lg) * wv_period(QW, gw) + word + l);
+    return d.tb + (size_t)it * WV_ITER + (uint32_t)(what + (strip & 1)) * WV_STREAM + ((at.y & 255u) + (uint32_t)l) * 8u;
 }
 
 }  // namespace

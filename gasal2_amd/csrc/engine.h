@@ -87,6 +87,16 @@ struct G2Dev {
     // ranked with their row (LOCAL: H <= 8191), 2: H alone.  When the census
     // refuses the score tables the lane kernels run the batch instead.
     uint32_t wave, wave_coop, wave64;
+    // WITH_TB on that path (wavetb.hip): the first wave64 sorted slots on 64
+    // lanes, the next wave16 (a multiple of four, or to the end) on 16, the rest
+    // on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
+    // and wv_strip (second best) max_tw words a slot, one per strip.
+    uint32_t wave16;
+    uint2 *wv_at;
+    uint32_t *wv_strip;
+    uint2 *wv_item;                  // second best: strips to recompute (k_second_strips), at most one per strip
+    uint64_t *wv_sec;                // and each slot's answer so far
+    uint32_t wv_walk;                // a wave walks each pair's path (k_wave_walk), else a lane (k_get_tb)
     // intra-pair wavefront for long pairs (LOCAL score + ends): pairs whose
     // shape passes wf_min_tw / wf_min_cells are sorted first and taken from an
     // atomic queue (aux[1], count in aux[2]) by the first wf_blocks blocks.
@@ -94,7 +104,7 @@ struct G2Dev {
     uint32_t *wf_scratch;            // per wavefront block: per pass 17 x 64 dwords of strip state
     uint32_t wf_stride;              // dwords per wavefront block
     uint32_t *wf_tb;                 // WITH_TB: tiles of the long pairs, per pair [strip][word] x 8 dwords
-    const uint64_t *wf_tbo;          // first 32-byte tile of each long pair in wf_tb
+    uint64_t *wf_tbo;                // first 32-byte tile of each long pair in wf_tb (claimed from aux[6..7])
     uint32_t *wf_tbh;                // checkpointed traceback of the long pairs: strip bottom rows
                                      // (wf_tb then holds the tiles' left column states); null: direction words
     // banded LOCAL (k_local_band): per-pair diagonal band [band_lo, band_hi]
@@ -125,6 +135,12 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
 
 // The DP of a batch on the packed one-wave path (d.wave, wave.hip).
 hipError_t g2_wave_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
+
+// LOCAL and GLOBAL WITH_TB on that path, the traceback's checkpoints included
+// (d.wave, wavetb.hip).
+hipError_t g2_wave_tb_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
+
+hipError_t g2_wave_walk(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
 
 // KSW in packed 16-bit strips (d.ksw_pk, ksw.hip).
 hipError_t g2_ksw_packed(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);

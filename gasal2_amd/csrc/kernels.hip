@@ -674,10 +674,10 @@ __global__ __launch_bounds__(256) void k_census(const uint32_t *__restrict__ pq,
     }
 }
 
-// Clears the batch's counters: the first four words of aux and the histogram.
+// Clears the batch's counters: the first eight words of aux and the histogram.
 __global__ __launch_bounds__(256) void k_zero_counters(uint32_t *aux, uint32_t *hist) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < 4) aux[k] = 0;
+    if (k < 8) aux[k] = 0;
     for (uint32_t i = k; i < (G2_SHAPE_BUCKETS + G2_SHAPE_ROWS) / 4; i += gridDim.x * blockDim.x)
         reinterpret_cast<uint4 *>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
 }
@@ -750,8 +750,16 @@ __device__ void wf_local(const G2Dev &d, const G2Scores &c, uint32_t census) {
         const int32_t npass = (TW + 63) / 64;
         const int32_t nblk = (C + WF_W - 1) / WF_W;
         // tiles per pair [strip][word] x 8 dwords
-        uint32_t *tbp = TB ? d.wf_tb + d.wf_tbo[pr] * 8 : nullptr;
-        uint32_t *thp = CK ? d.wf_tbh + d.wf_tbo[pr] * 8 : nullptr;
+        uint64_t tile0 = 0;   // claimed as the item is, every lane taking part
+        if (TB) {
+            const uint64_t got = atomicAdd(reinterpret_cast<unsigned long long *>(d.aux + 6),
+                                           l == 0 ? (unsigned long long)QW * (unsigned long long)TW : 0ull);
+            tile0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(got >> 32)) << 32 |
+                    (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)got);   // returns int: not to be sign-extended
+            if (l == 0) d.wf_tbo[pr] = tile0;
+        }
+        uint32_t *tbp = TB ? d.wf_tb + tile0 * 8 : nullptr;
+        uint32_t *thp = CK ? d.wf_tbh + tile0 * 8 : nullptr;
         WfBest lb = {0, 0x7FFFFFFF, 0x7FFFFFFF};
         for (int32_t b = 0; b < nblk; b++) {
             const int32_t c0 = b * WF_W;
@@ -2513,52 +2521,6 @@ __global__ __launch_bounds__(64) void k_ksw(G2Dev d, G2Scores c, int32_t w, int3
 }
 
 // --------------------------------------------------------------- get_tb -----
-// Recomputes one 8x8 tile's direction words (k_local_fast's sign-bit format)
-// from the checkpoints k_local_fast<.., CK> stored: the previous strip's
-// bottom row above the tile and the tile's left column state.  Same
-// recurrences and score tables (lut: the strip's eight rows, as k_local_fast
-// builds them), so the same words.
-// top: the row above, entry kk = (H at column kk - 1, E at column kk), so the
-// entry left of the tile's first column (the corner) comes with it; zero above
-// strip 0.  left: the left column state; lut: the strip's score tables (the
-// kernels store checkpoints only when the batch's nibble census allows tables).
-// The words hold the reference's nibbles (src/kernels/local_kernel_template.h
-// :45-60): [3] F continues (t <= f - extend), [2] E continues, [1:0] source:
-// diagonal 0 / 1 by the score's sign, F 3, E 2, ties in that order.
-__device__ __forceinline__ void ck_tile(const uint32_t *top, const uint32_t *left, uint32_t qword,
-                                        const uint32_t *lut, const G2Scores &c, uint32_t *ch) {
-    int32_t h[9], f[9];
-#pragma unroll
-    for (int m = 1; m < 9; m++) { h[m] = sx16(left[m - 1]); f[m] = (int32_t)left[m - 1] >> 16; }
-    const int32_t gapoe = c.gapoe, gape = c.gape;
-#pragma unroll
-    for (int kk = 0; kk < 8; kk++) {
-        const uint32_t qsh = kk < 7 ? (qword >> (26 - 4 * kk)) & 0x1Cu : (qword << 2) & 0x1Cu;
-        int32_t e = (int32_t)top[kk] >> 16;
-        int32_t p = sx16(top[kk]);
-        uint32_t dir = 0;
-#pragma unroll
-        for (int m = 1; m < 9; m++) {
-            const int32_t sc = __builtin_amdgcn_sbfe(lut[m - 1], qsh, 4);
-            const int32_t tmp = p + sc;
-            const int32_t hm = max(max(max(tmp, f[m]), e), 0);
-            const int32_t t = tmp - gapoe;
-            const int32_t fx = f[m] - gape, ex = e - gape;
-            const uint32_t na = (uint32_t)(tmp - hm);                       // sign: not from the diagonal
-            dir = __builtin_amdgcn_alignbit(dir, (uint32_t)t + ~(uint32_t)fx, 31);   // sign: fx >= t
-            dir = __builtin_amdgcn_alignbit(dir, (uint32_t)t + ~(uint32_t)ex, 31);   // sign: ex >= t
-            dir = __builtin_amdgcn_alignbit(dir, na, 31);
-            // low bit: from F (hm <= f) when not diagonal, else the mismatch flag (score < 0)
-            dir = __builtin_amdgcn_alignbit(dir, (na & ((uint32_t)hm + ~(uint32_t)f[m])) | (~na & (uint32_t)sc), 31);
-            f[m] = max(t, fx);
-            e = max(t, ex);
-            p = h[m];
-            h[m] = hm;
-        }
-        ch[kk] = dir;
-    }
-}
-
 // Word a of a packed sequence array through a 4-word register cache: the
 // aligned 16 bytes holding it are fetched when the walk first needs one of
 // them.  The arrays are 256-byte aligned with 4 words of slack past the last
@@ -2585,7 +2547,11 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     const uint32_t pr = d.perm[slot];
     // long pairs (sorted first) ran one wave per pair with per-pair tiles; the
     // lane path's groups count from the first slot after them
-    const uint32_t nlong = (LOCALT && d.wf_tb) ? d.aux[2] : 0u;
+    const uint32_t census = d.aux[0];
+    // every pair ran on the packed one-wave path (wavetb.hip)
+    const bool wv = d.wave && census_fast(census);
+    if (wv && d.wv_walk) return;   // walked by k_wave_walk
+    const uint32_t nlong = (LOCALT && d.wf_tb && !wv) ? d.aux[2] : 0u;
     const bool wfp = slot < nlong;
     const uint32_t rslot = slot - nlong;
     const uint32_t lane = rslot & (WAVE - 1), grp = rslot / WAVE;
@@ -2600,16 +2566,16 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     uint32_t bflag = 0;
     if (band && (d.band_flags[pr] & 8u)) { d.n_ops[pr] = 0; return; }
     // GLOBAL words are always in the sign-bit format (k_global)
-    const uint32_t census = d.aux[0];
     const bool lanefast = d.fast && d.enc_ok && census_fast(census);
     const bool fastfmt = !LOCALT || band || wfp || lanefast;
     // lane-path tiles of k_local_fast<.., CK> are recomputed from checkpoints
-    const bool ck = LOCALT && !band && !wfp && lanefast && d.tbh != nullptr;
+    const bool ck = LOCALT && !band && !wfp && !wv && lanefast && d.tbh != nullptr;
     // long pairs of k_local_fast's one-wave blocks with checkpoints (wf_local<.., CK>)
     const bool wck = LOCALT && wfp && d.wf_tbh != nullptr && census_fast(census);
     if (fused ? !ck : (ck && d.tb_fused)) return;   // walked by k_local_fast, or not fused there
     // recomputed tiles hold the reference's nibbles; stored sign-bit words are decoded
-    const bool decode = fastfmt && !ck && !wck;
+    const bool decode = fastfmt && !ck && !wck && !wv;
+    const uint2 wv_at = wv ? d.wv_at[pr] : make_uint2(0u, 0u);
     const uint32_t qw0 = d.qoff[pr] >> 3;
     const uint32_t *Qw = d.pq + qw0, *Tw = d.pt + (d.toff[pr] >> 3);
     uint4 q4 = {0u, 0u, 0u, 0u};   // recompute walks: cached query words
@@ -2644,18 +2610,18 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     while (!done) {
         const int32_t key = tile_key(i, j);
         if (key >= 0 && key != ch_key) {
-            const int32_t strip = key / QW, wv = key - strip * QW;
+            const int32_t strip = key / QW, word = key - strip * QW;
             const uint32_t *chunk = nullptr;
             if (band) {
                 int32_t wlo, whi;
                 band_words(strip, blo, bhi, QW, wlo, whi);
-                if (wv < wlo || wv >= whi || wv - wlo >= bbw) { bflag |= 2u; break; }   // walk left the band
-                if ((wv == wlo && wlo > 0) || (wv == whi - 1 && whi < QW)) bflag |= 1u;
-                chunk = d.tb + (d.band_tbo[pr] + (size_t)strip * bbw + (size_t)(wv - wlo)) * 8;
+                if (word < wlo || word >= whi || word - wlo >= bbw) { bflag |= 2u; break; }   // walk left the band
+                if ((word == wlo && wlo > 0) || (word == whi - 1 && whi < QW)) bflag |= 1u;
+                chunk = d.tb + (d.band_tbo[pr] + (size_t)strip * bbw + (size_t)(word - wlo)) * 8;
             } else if (wfp && !wck) {
-                chunk = d.wf_tb + (d.wf_tbo[pr] + (size_t)strip * QW + (size_t)wv) * 8;
+                chunk = d.wf_tb + (d.wf_tbo[pr] + (size_t)strip * QW + (size_t)word) * 8;
             }
-            if (ck || wck) {
+            if (ck || wck || wv) {
                 if (strip != lut_key) {   // the walk stays in one strip for several tiles
                     lut_key = strip;
                     const uint32_t gw = Tw[strip];
@@ -2665,33 +2631,37 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
                 uint32_t top[8], left[8];
                 if (ck) {
                     const TbView lv = tb_view(d, grp, lane), hv = tb_view(d, grp, lane, d.tbh);
-                    if (strip > 0) hv.load(strip - 1, wv, top);
-                    lv.load(strip, wv, left);
+                    if (strip > 0) hv.load(strip - 1, word, top);
+                    lv.load(strip, word, left);
+                } else if (wv) {
+                    if (strip > 0) tb_load(wv_tile(d, wv_at, QW, strip - 1, word, WV_BOTTOM), top);
+                    tb_load(wv_tile(d, wv_at, QW, strip, word, WV_LEFT), left);
                 } else {   // per pair [strip][word] x 8, H and E of the same column
                     const uint32_t *lp = d.wf_tb + d.wf_tbo[pr] * 8, *hp = d.wf_tbh + d.wf_tbo[pr] * 8;
                     if (strip > 0) {
                         uint32_t raw[8];
-                        tb_load(hp + ((size_t)(strip - 1) * QW + (size_t)wv) * 8, raw);
-                        const uint32_t corner = wv > 0 ? hp[((size_t)(strip - 1) * QW + (size_t)(wv - 1)) * 8 + 7] : 0u;
+                        tb_load(hp + ((size_t)(strip - 1) * QW + (size_t)word) * 8, raw);
+                        const uint32_t corner = word > 0 ? hp[((size_t)(strip - 1) * QW + (size_t)(word - 1)) * 8 + 7] : 0u;
 #pragma unroll
                         for (int k = 0; k < 8; k++)
                             top[k] = (raw[k] & 0xFFFF0000u) | ((k == 0 ? corner : raw[k - 1]) & 0xFFFFu);
                     }
-                    tb_load(lp + ((size_t)strip * QW + (size_t)wv) * 8, left);
+                    tb_load(lp + ((size_t)strip * QW + (size_t)word) * 8, left);
                 }
-                if (strip == 0) {
+                if (strip == 0) {   // the matrix's top boundary (GLOBAL: src/kernels/global.h:57-60)
 #pragma unroll
-                    for (int k = 0; k < 8; k++) top[k] = 0u;
+                    for (int k = 0; k < 8; k++)
+                        top[k] = LOCALT ? 0u : pk16(8 * word + k < 2 ? 0 : -(c.gapo + c.gape * (8 * word + k - 1)), NEG16);
                 }
-                ck_tile(top, left, seq_word4(d.pq, qw0 + (uint32_t)wv, q4, q4_key), lut, c, ch);
+                ck_tile<LOCALT>(top, left, seq_word4(d.pq, qw0 + (uint32_t)word, q4, q4_key), lut, c, ch);
             } else if (chunk) {
                 tb_load(chunk, ch);
             } else {
-                tb_view(d, grp, lane).load(strip, wv, ch);
+                tb_view(d, grp, lane).load(strip, word, ch);
             }
             ch_key = key;
         }
-        if (LOCALT && (ck || wck)) {
+        if (LOCALT && (ck || wck || wv)) {
             // recomputed tiles: reference nibbles, and a LOCAL walk stays inside
             // the matrix, so a step reads the column's word (re-selected only on
             // a column move) and the tile changes when i >> 3 or j >> 3 does
@@ -2787,8 +2757,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     // score table of each target nibble for the tile recompute (one per block,
     // built before any thread leaves)
     __shared__ uint32_t lut16[16];
-    if (LOCALT) {
-        if (threadIdx.x < 16) lut16[threadIdx.x] = score_lut(c, c.has_np ? -c.np : 0, d.aux[0], threadIdx.x);
+    if (LOCALT || d.wave) {
+        if (threadIdx.x < 16)
+            lut16[threadIdx.x] = LOCALT ? score_lut(c, c.has_np ? -c.np : 0, d.aux[0], threadIdx.x)
+                                        : score_lut<true>(c, 0, d.aux[0], threadIdx.x);
         __syncthreads();
     }
     tb_walk<LOCALT>(d, c, blockIdx.x * blockDim.x + threadIdx.x, lut16, false);
@@ -2945,10 +2917,11 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             break;
         case A_LOCAL:
             if (d.wave) {
-                const hipError_t e = g2_wave_run(sc, op, d, s);
+                const hipError_t e = tb ? g2_wave_tb_run(sc, op, d, s) : g2_wave_run(sc, op, d, s);
                 if (e != hipSuccess) return e;
                 // a batch without score tables keeps one wave per long pair
-                if (d.wf_blocks) k_local_fast<S_WITHOUT_START, false><<<dim3(groups + d.wf_blocks), blk, 0, s>>>(d, sc);
+                if (d.wf_blocks && tb) k_local_fast<S_WITH_TB, false><<<dim3(groups + d.wf_blocks), blk, 0, s>>>(d, sc);
+                else if (d.wf_blocks) k_local_fast<S_WITHOUT_START, false><<<dim3(groups + d.wf_blocks), blk, 0, s>>>(d, sc);
             } else if (d.fast && d.pk2) {   // two pairs per lane: half the lane-path blocks
                 const dim3 g2((groups + 1) / 2), g2w((groups + 1) / 2 + d.wf_blocks);
                 if (op.start == S_WITH_TB) {
@@ -2994,7 +2967,7 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             break;
         case A_GLOBAL:
             if (d.wave) {
-                const hipError_t e = g2_wave_run(sc, op, d, s);
+                const hipError_t e = tb ? g2_wave_tb_run(sc, op, d, s) : g2_wave_run(sc, op, d, s);
                 if (e != hipSuccess) return e;
             } else if (d.fast) {
                 if (tb) k_global<true, true><<<grid, blk, 0, s>>>(d, sc);
@@ -3072,6 +3045,10 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
     if (timing) (void)hipEventRecord(tm->ev[3], s);
     // 5. traceback (src/gasal_align.h:45-53,60-68)
     if (tb) {
+        if (d.wave && d.wv_walk) {
+            const hipError_t e = g2_wave_walk(sc, op, d, s);
+            if (e != hipSuccess) return e;
+        }
         if (op.algo == A_LOCAL) k_get_tb<true><<<grid, blk, 0, s>>>(d, sc);
         else if (op.algo == A_GLOBAL) k_get_tb<false><<<grid, blk, 0, s>>>(d, sc);
         else k_no_tb<<<nb256, 256, 0, s>>>(d);

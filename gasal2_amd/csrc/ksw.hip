@@ -39,9 +39,6 @@
 namespace {
 
 typedef unsigned short pu16x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ pk16x2 pmaxu(pk16x2 a, pk16x2 b) {
-    return __builtin_bit_cast(pk16x2, __builtin_elementwise_max(__builtin_bit_cast(pu16x2, a), __builtin_bit_cast(pu16x2, b)));
-}
 __device__ __forceinline__ pk16x2 pmin(pk16x2 a, pk16x2 b) { return __builtin_elementwise_min(a, b); }
 // 1 in each half that is not 0
 __device__ __forceinline__ pk16x2 nonzero_one(pk16x2 v) {
@@ -55,13 +52,6 @@ __device__ __forceinline__ pk16x2 times8(pk16x2 v) {
     return as_pk(r);
 }
 __device__ __forceinline__ uint32_t or3(uint32_t a, uint32_t b, uint32_t c) { return a | b | c; }
-__device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
-
-__device__ __forceinline__ int32_t wave_max(int32_t v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
-    return __builtin_amdgcn_readfirstlane(v);
-}
 
 // One lane per pair, strips 2k and 2k + 1 in the low and high halves, the high
 // one a column behind.
@@ -96,8 +86,8 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
     int32_t bv = h0, bi = -1, bj = -1;      // the reference's max, max_i, max_j
     int32_t gs = -1, gi = -1;               // gscore, max_ie
     uint32_t redo = 0;                      // the pair needs the row by row kernel
-    const int32_t TWm = wave_max(TW);
-    int32_t ws = 0, we = wave_max(QW);      // the wave's words
+    const int32_t TWm = wave_max<1>(TW);
+    int32_t ws = 0, we = wave_max<1>(QW);      // the wave's words
     for (int32_t s0 = 0; s0 < TWm; s0 += 2) {
         const bool act = s0 < TW;
         const int32_t RL = 8 * s0, RH = RL + 8;   // first rows of the two strips
@@ -264,8 +254,8 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
         const bool dead = !more || (last_w < 0 && !lb);
         const int32_t lo = dead ? 0x7FFF : (lb ? 0 : max(first_w - 1, 0));
         const int32_t hi = dead ? 0 : min(QW, last_w + 6);
-        ws = max(ws, -wave_max(-lo));
-        we = wave_max(hi);
+        ws = max(ws, -wave_max<1>(-lo));
+        we = wave_max<1>(hi);
         if (we <= ws) break;
     }
     if (!ok) return;

@@ -25,7 +25,7 @@ constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
 uint8_t *g_scratch_ptr[MAX_DEVICES] = {};   // device address of `scratch` on each device
 
-constexpr uint32_t AUX_BAD = 16;   // aux word counting rejected pairs (g2_run uses words 0..3)
+constexpr uint32_t AUX_BAD = 16;   // aux word counting rejected pairs (g2_run uses words 0..7)
 
 // Copies offsets, lengths and operations into the scratch; a pair whose
 // sequence does not lie inside its batch at a multiple of 8 bases, or is

@@ -18,6 +18,7 @@
 #include <mutex>
 #include <algorithm>
 #include <cmath>
+#include <functional>
 
 // ------------------------------------------------------------ globals ------
 // An order chain (the batch order below).
@@ -154,7 +155,12 @@ struct Impl {
     size_t wf_tb_bytes = 0;
     uint64_t *wf_tbo = nullptr;
     size_t wf_tbo_bytes = 0;
-    std::vector<uint64_t> h_wf_tbo;
+    uint2 *wv_at = nullptr;          // packed one-wave traceback path: pairs' places, strips' records
+    uint32_t *wv_strip = nullptr;
+    uint2 *wv_item = nullptr;
+    uint64_t *wv_sec = nullptr;
+    size_t wv_at_bytes = 0, wv_strip_bytes = 0, wv_item_bytes = 0, wv_sec_bytes = 0;
+    std::vector<uint32_t> h_keys, h_khist;
     std::vector<int32_t> h_lo, h_hi;
     std::vector<uint32_t> h_bw;
     std::vector<uint64_t> h_tbo;
@@ -849,7 +855,7 @@ static void impl_free(Impl *m) {
     order_forget(m);
     if (m->ev_h2d) (void)hipEventDestroy(m->ev_h2d);
     if (m->ev_dev) (void)hipEventDestroy(m->ev_dev);
-    void *ptrs[] = {m->qpan, m->tpan, m->tb_gbase, m->tb_gqw, m->wf_tb, m->wf_tbo, m->band_wres, m->band_lo, m->band_hi, m->band_bw, m->band_tbo, m->band_flags, m->sub_u32, m->sub_res,
+    void *ptrs[] = {m->qpan, m->tpan, m->tb_gbase, m->tb_gqw, m->wf_tb, m->wf_tbo, m->wv_at, m->wv_strip, m->wv_item, m->wv_sec, m->band_wres, m->band_lo, m->band_hi, m->band_bw, m->band_tbo, m->band_flags, m->sub_u32, m->sub_res,
                     m->sub_nops, m->sub_cigar,
                     m->keys, m->perm, m->hist, m->bnd, m->tb, m->eh,
                     m->nops, m->cigar, m->cigar_q, m->scratch_i32, m->aux, m->wf};
@@ -989,6 +995,72 @@ uint32_t g2_wave_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_
     if (op.algo == LOCAL) return hmax <= 8191 ? 1 : (hmax <= 32000 ? 2 : 0);
     const int64_t low = 3ll * sc.gapoe + sc.gape * (16ll * std::max(qw, tw) + 64) + 2 * down;
     return hmax <= 32000 && low <= 29000 ? 1 : 0;
+}
+
+// WITH_TB on that path (wavetb.hip): LOCAL and GLOBAL whose values fit 16 bits
+// with the reference's negative E and F, ranked cells, no empty sequence.
+bool wave_tb_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw, int32_t fast) {
+    if (op.start != WITH_TB || (op.algo != LOCAL && op.algo != GLOBAL) || !g_tb_ckpt || g_tb_fused) return false;
+    if (sc.gapoe > 16000 || sc.gapo < 0 || sc.gape < 0 || tw >= 1u << 18) return false;
+    G2Opts plain = op;
+    plain.start = WITHOUT_START;
+    plain.second = 0;
+    return g2_wave_fits(plain, sc, qw, tw, fast) == 1;
+}
+
+// Iterations of a pair on gw lanes of that path.
+uint64_t wave_tb_iters(uint32_t qw, uint32_t tw, uint32_t gw) {
+    return (uint64_t)((tw + 2 * gw - 1) / (2 * gw)) * std::max(qw, gw + 1) + gw;
+}
+
+// Lanes of a pair: 4 unless its iterations there would outlast the batch's
+// share of a SIMD (work: wave-iterations of the batch on 4 lanes; 1.5: a wave
+// alone on a SIMD against its share of a full one), else the least of 16 and
+// 64 that would not, else what is fewest iterations.
+uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double work) {
+    const double share = work / (g2_cu_count() * 4.0 + 1.0) / 1.5;
+    uint32_t best = 4;
+    for (uint32_t gw : {4u, 16u, 64u}) {
+        const uint64_t its = wave_tb_iters(qw, tw, gw);
+        if ((double)its <= share) return gw;
+        if (its < wave_tb_iters(qw, tw, best)) best = gw;
+    }
+    return best;
+}
+
+// Whether LOCAL WITH_TB runs there: padded cells, the longest pair's, and the
+// path's wave-iterations on 4 lanes.  The lane kernels (two pairs a lane) are
+// bound by the longest pair's serial time, part of which other launches on the
+// device can hide, and their rate; that path by its rate, the second best's
+// strips included.  100-300 x 100-400 bases with second best, lanes / that path:
+// 30,000 pairs 6.2 / 1.8 ms, 100,000 6.4 / 3.5, 300,000 11.0 / 9.3 alone and 7.9 /
+// 8.2 among other passes, 900,000 19.5 / 26.8; 150 x 250 without: 100,000 pairs
+// 3.0 / 2.0, 300,000 5.7 / 5.0, 1,000,000 15.7 / 17.0.  GLOBAL always does: its
+// lanes store direction words in 32 bits, 900,000 pairs 26.4 / 23.9 ms.
+bool wave_tb_pays(const G2Opts &op, double cells, double longest, double work) {
+    if (op.algo == GLOBAL) return true;
+    return work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
+}
+
+// Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb): the
+// longest path's serial time (1.6 us a cell on a lane, 0.1 on a wave) against
+// the sum's (11 ps a cell on lanes, 62 on waves).  Lanes / waves: 64 pairs of
+// 100-300 bases 486 / 53 us, 51,000 617 / 638, 120,000 727 / 1432; 50,000 pairs
+// of 50-5000 bases 8.7 / 1.6 ms.
+bool wave_walk_pays(double sum, double longest) { return 40e-6 + 51e-12 * sum < 1.6e-6 * longest; }
+
+// Shape buckets as the device sorts by them (k_keys), and a bucket's largest x.
+uint32_t shape8(uint32_t x) {
+    if (x < 128u) return x;
+    const uint32_t e = 31u - (uint32_t)__builtin_clz(x);
+    const uint32_t v = 128u + (e - 7u) * 16u + ((x >> (e - 4u)) & 15u);
+    return v > 255u ? 255u : v;
+}
+uint32_t shape8_edge(uint32_t v) {
+    if (v < 128u) return v;
+    if (v == 255u) return 0xFFFFFFFFu;
+    const uint32_t e = 7u + (v - 128u) / 16u, mant = (v - 128u) % 16u;
+    return ((17u + mant) << (e - 4u)) - 1u;
 }
 
 // Whether that path beats the lane kernels on a batch.  total and longest:
@@ -1353,6 +1425,67 @@ G2Opts opts_of(const Parameters *p, const gasal_gpu_storage_t *s) {
     return o;
 }
 
+// The packed one-wave traceback path's launch (d.wave64, d.wave16) and the most
+// iterations its waves can claim together: the batch's shapes in the device's
+// sorted order (k_keys), each bucket at its largest shape, every wave at its
+// longest pair's.
+uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht, uint32_t n, uint32_t qw, uint32_t tw) {
+    std::vector<std::pair<uint32_t, uint32_t>> runs;   // key, pairs, in descending key order
+    auto key_of = [&](uint32_t k) -> uint32_t {
+        const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
+        const bool lng = d.wf_blocks > 0 && kt >= d.wf_min_tw && (uint64_t)kq * kt * 64u >= (uint64_t)d.wf_min_cells;
+        return (lng ? 0x10000u : 0u) | (shape8(kq) << 8) | shape8(kt);
+    };
+    if (n <= 8192) {
+        m->h_keys.resize(n);
+        for (uint32_t k = 0; k < n; k++) m->h_keys[k] = key_of(k);
+        std::sort(m->h_keys.begin(), m->h_keys.end(), std::greater<uint32_t>());
+        for (uint32_t k = 0; k < n; k++) {
+            if (k == 0 || m->h_keys[k] != m->h_keys[k - 1]) runs.push_back({m->h_keys[k], 0});
+            runs.back().second++;
+        }
+    } else {
+        m->h_khist.assign(G2_SHAPE_BUCKETS, 0u);
+        for (uint32_t k = 0; k < n; k++) m->h_khist[key_of(k)]++;
+        for (uint32_t key = G2_SHAPE_BUCKETS; key-- > 0;)
+            if (m->h_khist[key]) runs.push_back({key, m->h_khist[key]});
+    }
+    auto q_of = [&](uint32_t key) { return std::min(shape8_edge((key >> 8) & 255u), qw); };
+    auto t_of = [&](uint32_t key) { return std::min(shape8_edge(key & 255u), tw); };
+    double work = 0;
+    for (const auto &r : runs) work += (double)r.second * wave_tb_iters(q_of(r.first), t_of(r.first), 4) / 16.0;
+    uint32_t n64 = 0, n16 = 0;
+    for (const auto &r : runs) {
+        const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), work);
+        if (lanes == 64) n64 += r.second;
+        if (lanes == 16) n16 += r.second;
+    }
+    n16 = std::min((n16 + 3) & ~3u, n - n64);
+    d.wave64 = n64;
+    d.wave16 = n16;
+    uint64_t total = 0, longest = 0;
+    uint32_t slot = 0, room = 0;
+    for (const auto &r : runs) {
+        uint32_t c = r.second, gw = 0;
+        uint64_t its = 0;
+        while (c) {
+            if (!room) {
+                total += longest;
+                longest = 0;
+                room = slot < n64 ? 1 : (slot < n64 + n16 ? 4 : 16);
+            }
+            const uint32_t g = slot < n64 ? 64 : (slot < n64 + n16 ? 16 : 4);
+            if (g != gw) its = wave_tb_iters(q_of(r.first), t_of(r.first), gw = g);
+            longest = std::max(longest, its);
+            const uint32_t take = std::min(c, room);
+            c -= take;
+            room -= take;
+            slot += take;
+        }
+    }
+    return total + longest;
+}
+
 // Sizes the workspace for this batch and fills the device view.
 struct PrepExtra {
     const uint32_t *hq = nullptr, *ht = nullptr;   // host lengths of the pairs run (default: the storage's)
@@ -1452,6 +1585,34 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
 
     const G2Scores &sc = g_scores;
     g2_choose_fast(d, op, sc, qw, tw);
+    // WITH_TB on the packed one-wave path (wavetb.hip); thresholds set by the
+    // caller or the tuner keep the kernels they switch.  Its checkpoints may
+    // take half of the device memory free now (this storage's own tile buffer
+    // counted as free: it is reused): about 64 B per tile and 5 KB a pair.
+    bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
+                   wave_tb_fits(op, sc, qw, tw, d.fast);
+    uint64_t wave_strips = 0, path_sum = 0, path_max = 0;
+    if (wave_tb) {
+        uint64_t tiles = 0, longest = 0, work = 0;
+        uint32_t least = 0xFFFFFFFFu;
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
+            least = std::min(least, std::min(hq[k], ht[k]));
+            tiles += (uint64_t)kq * kt;
+            longest = std::max(longest, (uint64_t)kq * kt);
+            work += wave_tb_iters(kq, kt, 4);
+            wave_strips += kt;
+            const uint32_t path = op.algo == LOCAL ? std::min(hq[k], ht[k]) : std::max(hq[k], ht[k]);
+            path_sum += path;
+            path_max = std::max<uint64_t>(path_max, path);
+        }
+        size_t free_b = 0, total_b = 0;
+        wave_tb = least > 0 &&
+                  (g2_get_dispatch() == 3 || wave_tb_pays(op, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
+                  hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+                  tiles * 90 + (uint64_t)n * 5000 <= ((uint64_t)free_b + m->tb_bytes) / 2;
+    }
+    uint64_t wf_bytes = 0;   // wave_tb: direction words of the long pairs, within the tile buffer
     // Long LOCAL pairs (score and ends only) run one wave per pair.  The
     // device applies the same shape test in k_keys and also needs the nibble
     // census to allow the score tables; the host count only sizes the launch.
@@ -1477,6 +1638,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 }
         }
         switched |= tuned;
+        wave_tb = wave_tb && !tuned;
         // the small-batch rule yields to user and tuned thresholds
         const bool few = g2_get_dispatch() == 0 && !g_wf_user && !tuned &&
                          (uint64_t)n <= (uint64_t)g2_cu_count() * (op.start == WITH_TB ? WF_FEW_PER_CU_TB : WF_FEW_PER_CU);
@@ -1485,7 +1647,6 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         d.wf_min_cells = all ? 0u : min_cells;
         uint32_t ltw = 0, lqw = 0, sq = 0, st = 0;
         const bool wtb = op.start == WITH_TB;
-        if (wtb) m->h_wf_tbo.resize(n);
         uint64_t wtot = 0;   // 32-byte tiles of the long pairs
         // no pair can pass the shape test when the largest shapes do not
         const bool any_long = tw >= d.wf_min_tw && (uint64_t)qw * tw * 64u >= (uint64_t)d.wf_min_cells;
@@ -1495,7 +1656,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 nlong++;
                 ltw = std::max(ltw, kt);
                 lqw = std::max(lqw, kq);
-                if (wtb) { m->h_wf_tbo[k] = wtot; wtot += (uint64_t)kq * kt; }
+                if (wtb) wtot += (uint64_t)kq * kt;
             } else {
                 sq = std::max(sq, kq);
                 st = std::max(st, kt);
@@ -1513,7 +1674,11 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 d.wf_stride = 0;
                 d.wf_scratch = nullptr;
             }
-            if (wtb) {   // per-pair direction tiles (or checkpoints) of the long pairs and their offsets
+            if (wave_tb) {   // run only when the census refuses the score tables
+                wf_bytes = wtot * 32;
+                ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
+                d.wf_tbo = m->wf_tbo;
+            } else if (wtb) {   // per-pair direction tiles (or checkpoints) of the long pairs; the waves claim their places
                 // checkpoints take twice the bytes of direction words: only while
                 // they fit in 80% of the device memory free now (this storage's
                 // own buffer counted as free: it is reused)
@@ -1527,7 +1692,6 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                                      32767u;
                 ensure(m->wf_tb, m->wf_tb_bytes, (size_t)wtot * 32 * (wck ? 2 : 1) + 256);
                 ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
-                G2_CHECK(hipMemcpyAsync(m->wf_tbo, m->h_wf_tbo.data(), (size_t)n * 8, hipMemcpyHostToDevice, s->str));
                 d.wf_tb = m->wf_tb;
                 d.wf_tbo = m->wf_tbo;
                 if (wck) d.wf_tbh = m->wf_tb + wtot * 8;
@@ -1542,7 +1706,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         d.ksw_pk = 1;
     // Transposed sequence panels for the fast LOCAL and KSW lane path (k_panel):
     // groups after the long pairs, eq query words and et target words each.
-    if (g_panels && (d.ksw_pk || (d.fast && op.algo == LOCAL)) && !px.banded && n > nlong) {
+    if (g_panels && (d.ksw_pk || (d.fast && op.algo == LOCAL)) && !px.banded && !wave_tb && n > nlong) {
         const uint64_t lgroups = ((uint64_t)(n - nlong) + 63) / 64;
         ensure(m->qpan, m->qpan_bytes, (size_t)(lgroups * eq * 256) + 256);
         ensure(m->tpan, m->tpan_bytes, (size_t)(lgroups * et * 256) + 256);
@@ -1551,6 +1715,23 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         d.qpan_w = eq;
         d.tpan_w = et;
     }
+    // The packed one-wave path's checkpoints and the direction words of the
+    // kernels that run when the census refuses the score tables share one buffer.
+    uint64_t wave_bytes = 0;
+    if (wave_tb) {
+        wave_bytes = wave_tb_plan(m, d, hq, ht, n, qw, tw) * 8192;
+        ensure(m->wv_at, m->wv_at_bytes, (size_t)n * 8);
+        d.wv_at = m->wv_at;
+        d.wv_walk = wave_walk_pays((double)path_sum, (double)path_max);
+        if (op.second) {
+            ensure(m->wv_strip, m->wv_strip_bytes, (size_t)n * tw * 4);
+            ensure(m->wv_item, m->wv_item_bytes, (size_t)wave_strips * 8);
+            ensure(m->wv_sec, m->wv_sec_bytes, (size_t)n * 8);
+            d.wv_strip = m->wv_strip;
+            d.wv_item = m->wv_item;
+            d.wv_sec = m->wv_sec;
+        }
+    }
     // direction tiles of the one-lane-per-pair kernels: groups after the long pairs
     if (tb_dp && !px.banded) {
         const uint64_t lgroups = ((uint64_t)(n - nlong) + 63) / 64;
@@ -1558,7 +1739,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         // Checkpointed traceback: two regions of the tile layout (left column
         // states, strip bottom rows) instead of direction words.  Stored
         // states are 16-bit, so H must fit: H <= match * min(Lq, Lt).
-        const bool ck = g_tb_ckpt && op.algo == LOCAL && op.start == WITH_TB && d.fast &&
+        const bool ck = g_tb_ckpt && !wave_tb && op.algo == LOCAL && op.start == WITH_TB && d.fast &&
                         (uint64_t)std::max(sc.match, 0) * 8u * std::min(eq, et) <= 32767u &&
                         (uint64_t)sc.gapoe + (uint64_t)std::max(std::max(sc.mismatch, sc.has_np ? sc.np : 0), 0) <= 32767u;
         const uint64_t nreg = ck ? 2 : 1;
@@ -1574,25 +1755,14 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 one = nreg * one_size <= ((uint64_t)free_b + m->tb_bytes) / 2;
         }
         if (one) {
-            ensure(m->tb, m->tb_bytes, (size_t)(nreg * one_size) + 256);
+            ensure(m->tb, m->tb_bytes, (size_t)std::max(nreg * one_size + wf_bytes, wave_bytes) + 256);
+            if (wf_bytes) d.wf_tb = m->tb + one_size / 4;
             if (ck) d.tbh = m->tb + one_size / 4;
         } else {
             // Per-group regions.  The device orders the lane-path pairs by
             // descending shape bucket (k_keys), so the buckets falling in each
             // 64-slot group are fixed; each group gets the largest bucket
             // edges among them.
-            auto shape8 = [](uint32_t x) -> uint32_t {
-                if (x < 128u) return x;
-                uint32_t e = 31u - (uint32_t)__builtin_clz(x);
-                uint32_t v = 128u + (e - 7u) * 16u + ((x >> (e - 4u)) & 15u);
-                return v > 255u ? 255u : v;
-            };
-            auto edge8 = [](uint32_t v) -> uint32_t {   // largest x with shape8(x) == v
-                if (v < 128u) return v;
-                if (v == 255u) return 0xFFFFFFFFu;
-                uint32_t e = 7u + (v - 128u) / 16u, mant = (v - 128u) % 16u;
-                return ((17u + mant) << (e - 4u)) - 1u;
-            };
             m->h_hist.assign(1u << 16, 0u);
             const bool wfa = d.wf_blocks > 0;
             for (uint32_t k = 0; k < n; k++) {
@@ -1607,7 +1777,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             for (int32_t key = (1 << 16) - 1; key >= 0; key--) {
                 uint32_t c = m->h_hist[key];
                 if (!c) continue;
-                const uint32_t qe = std::min(edge8((uint32_t)key >> 8), eq), te = std::min(edge8((uint32_t)key & 255u), et);
+                const uint32_t qe = std::min(shape8_edge((uint32_t)key >> 8), eq), te = std::min(shape8_edge((uint32_t)key & 255u), et);
                 const uint64_t g0 = slot / 64, g1 = (slot + c - 1) / 64;
                 for (uint64_t g = g0; g <= g1 && g < lgroups; g++) {
                     m->h_gqw[g] = std::max(m->h_gqw[g], qe);
@@ -1620,7 +1790,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 m->h_gbase[g] = tot;
                 tot += (uint64_t)gtw[g] * m->h_gqw[g] * 64 * 8;
             }
-            ensure(m->tb, m->tb_bytes, (size_t)(nreg * tot) * 4 + 256);
+            ensure(m->tb, m->tb_bytes, (size_t)std::max(nreg * tot * 4 + wf_bytes, wave_bytes) + 256);
+            if (wf_bytes) d.wf_tb = m->tb + tot;
             if (ck) d.tbh = m->tb + tot;
             ensure(m->tb_gbase, m->tb_gbase_bytes, (size_t)lgroups * 8 + 256);
             ensure(m->tb_gqw, m->tb_gqw_bytes, (size_t)lgroups * 4 + 256);
@@ -1637,8 +1808,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         s->packed_tb_matrix_size = m->tb_bytes / 16;
     }
     g2_choose_packed(d, op, sc, eq, et, px.banded);
-    if (!px.banded) d.wave = g2_wave_fits(op, sc, qw, tw, d.fast);
-    if (d.wave) {
+    if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
+    if (d.wave && !wave_tb) {
         // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
         const bool mixed = op.algo == LOCAL && op.start == WITHOUT_START;
         uint64_t total = 0, longest = 0, steps = 0;
@@ -1692,7 +1863,7 @@ void upload_async(gasal_gpu_storage_t *s, uint32_t n, Parameters *params) {
 // trigger a new capture.  The program holds kernels only (no memset or copy
 // nodes).  Timed runs (per-stage events) launch eagerly.
 hipError_t launch_program(Impl *m, const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t st) {
-    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh ? 4 : 0);
+    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh || (d.wave && op.start == WITH_TB) ? 4 : 0);
     if (!g_graph_mode || m->tm.enabled) return g2_run(sc, op, d, st, &m->tm);
     const bool same = m->g_valid && memcmp(&m->g_dev, &d, sizeof(d)) == 0 && memcmp(&m->g_sc, &sc, sizeof(sc)) == 0 &&
                       memcmp(&m->g_op, &op, sizeof(op)) == 0;

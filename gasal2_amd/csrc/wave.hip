@@ -38,33 +38,6 @@ constexpr int PW_WAVES = 4;   // per block
 enum { PW_LOCAL, PW_GLOBAL, PW_SEMI };
 enum { PW_FORWARD, PW_LOCAL_REVERSE, PW_SEMI_REVERSE };   // how a run reads its sequences
 
-// the previous lane's v within the group; the group's first lane: first
-template <int GW>
-__device__ __forceinline__ uint32_t from_above(uint32_t first, uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, GW == 16 ? 0x111 : 0x138, 0xF, 0xF, false);
-}
-// maximum over the wave of a value that is uniform within 16-lane rows
-__device__ __forceinline__ int32_t wave_max(int32_t v) {
-    v = max(v, __shfl_xor(v, 16));
-    v = max(v, __shfl_xor(v, 32));
-    return __builtin_amdgcn_readfirstlane(v);
-}
-__device__ __forceinline__ pk16x2 pmaxu(pk16x2 a, pk16x2 b) {
-    typedef unsigned short pu16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(pk16x2, __builtin_elementwise_max(__builtin_bit_cast(pu16x2, a), __builtin_bit_cast(pu16x2, b)));
-}
-// 0xFFFF in each half that is not 0 (written out: the compiler makes compares
-// and selects per half of it)
-__device__ __forceinline__ uint32_t nonzero_mask(pk16x2 v) {
-    uint32_t one, m;
-    asm("v_pk_min_u16 %0, %1, 1 op_sel_hi:[1,0]" : "=v"(one) : "v"(as_u32(v)));
-    asm("v_pk_sub_i16 %0, 0, %1" : "=v"(m) : "v"(one));
-    return m;
-}
-__device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) { return (a & mask) | (b & ~mask); }
-__device__ __forceinline__ pk16x2 set_lo(pk16x2 v, int32_t x) { return as_pk(bits_of(0xFFFFu, (uint32_t)x, as_u32(v))); }
-__device__ __forceinline__ pk16x2 set_hi(pk16x2 v, int32_t x) { return as_pk(pack_lo(as_u32(v), (uint32_t)x)); }
-
 // One DP over a group's pair (uniform within the group).
 struct PwPair {
     const uint32_t *q, *t;   // forward, semi reverse: the first word; LOCAL reverse: the last word
