@@ -45,7 +45,7 @@ def build_synth():
 def build_lib():
     out = os.path.join(HERE, "libgasal2_amd.so")
     objs, cmds = [], []
-    for src in ("kernels.hip", "wave.hip", "wavetb.hip", "ksw.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
+    for src in ("kernels.hip", "wave.hip", "wavetb.hip", "ksw.hip", "banded.hip", "band.hip", "noalloc.hip", "runtime.cpp", "stream.cpp", "sam.cpp"):
         obj = os.path.join(CSRC, "_build", src + ".o")
         os.makedirs(os.path.dirname(obj), exist_ok=True)
         lang = ["-x", "hip"] if src.endswith(".hip") else []

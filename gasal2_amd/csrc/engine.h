@@ -68,6 +68,7 @@ struct G2Dev {
     uint32_t eh_cols;
     int32_t ksw16;                   // KSW rows as packed uint16 (H, E): values fit 16 bits
     uint32_t ksw_pk;                 // KSW in packed strips (ksw.hip); k_ksw runs the pairs it lists in keys (aux[3])
+    uint32_t band_pk;                // BANDED in packed 16-bit halves (banded.hip)
     uint32_t *aux;                   // small device counters (work queue etc.)
     uint32_t *sink;                  // 4 KiB a kernel may write discarded records to (never read)
     // score-table kernels (k_local_fast, k_global / k_semi LUT variants): 0 =
@@ -141,6 +142,9 @@ hipError_t g2_wave_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hip
 hipError_t g2_wave_tb_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
 
 hipError_t g2_wave_walk(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
+
+// BANDED in packed 16-bit halves (d.band_pk, banded.hip).
+hipError_t g2_banded_packed(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);
 
 // KSW in packed 16-bit strips (d.ksw_pk, ksw.hip).
 hipError_t g2_ksw_packed(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t stream);

@@ -2998,7 +2998,12 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
             }
             break;
         case A_BANDED:
-            if (d.fast) k_banded<true><<<grid, blk, 0, s>>>(d, sc, op.k_band >> 3);          // src/gasal_align.h:80
+            if (d.band_pk) {
+                const hipError_t e = g2_banded_packed(sc, op, d, s);
+                if (e != hipSuccess) return e;
+            } else if (d.fast) {
+                k_banded<true><<<grid, blk, 0, s>>>(d, sc, op.k_band >> 3);                  // src/gasal_align.h:80
+            }
             k_banded<false><<<grid, blk, 0, s>>>(d, sc, op.k_band >> 3);
             break;
         case A_KSW:

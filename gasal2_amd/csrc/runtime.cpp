@@ -1698,6 +1698,13 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             }
         }
     }
+    // BANDED in packed halves: E and F are held at or above 0, so every value
+    // lies in [-open, H], and ranked cells need H <= 8191; steps are held in 16
+    // bits.
+    if (op.algo == BANDED && d.fast && g_pk16_mode && sc.gape >= 0 && sc.gape <= 16000 && sc.gapoe >= 0 && sc.gapoe <= 16000 &&
+        (int64_t)std::max({sc.match, -sc.mismatch, sc.has_np ? -sc.np : 0, 0}) * 8 * std::min(qw, tw) <= 8191 &&
+        8ull * qw + 8 <= 65535)
+        d.band_pk = 1;
     // KSW in packed strips: the reference's form (no band, no z-drop), ranked
     // cells (H <= 4095), an end bonus that a gap open covers (ksw.hip).
     if (op.algo == KSW && d.fast && g_pk16_mode && op.ksw_w < 0 && op.ksw_zdrop <= 0 && ksw_hmax <= 4095 && sc.gapo >= 0 &&
@@ -1863,7 +1870,7 @@ void upload_async(gasal_gpu_storage_t *s, uint32_t n, Parameters *params) {
 // trigger a new capture.  The program holds kernels only (no memset or copy
 // nodes).  Timed runs (per-stage events) launch eagerly.
 hipError_t launch_program(Impl *m, const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t st) {
-    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh || (d.wave && op.start == WITH_TB) ? 4 : 0);
+    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16 || d.band_pk) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh || (d.wave && op.start == WITH_TB) ? 4 : 0);
     if (!g_graph_mode || m->tm.enabled) return g2_run(sc, op, d, st, &m->tm);
     const bool same = m->g_valid && memcmp(&m->g_dev, &d, sizeof(d)) == 0 && memcmp(&m->g_sc, &sc, sizeof(sc)) == 0 &&
                       memcmp(&m->g_op, &op, sizeof(op)) == 0;
