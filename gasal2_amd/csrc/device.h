@@ -178,14 +178,22 @@ __device__ __forceinline__ void ck_tile(const uint32_t *top, const uint32_t *lef
 // is a log of its iterations: 8 KiB each, four streams of one 32-byte record a
 // lane -- left column state of the low and the high strip, bottom row of the
 // low and the high strip -- so that every store of a wave covers whole lines.
-// at: the pair's first iteration, first lane | log2(lanes of its group) << 8.
+// at: the pair's first iteration, first lane | log2(lanes of its group) << 8; for
+// a pair on a block's four waves 8 there, | iterations of a wave's region << 12
+// (the four regions follow each other, passes dealt to them in turn).
 constexpr uint32_t WV_STREAM = WAVE * 8, WV_ITER = 4 * WV_STREAM;   // dwords
 enum { WV_LEFT = 0, WV_BOTTOM = 2 };
-// iterations from a group's pass to its next one: its words, or the lanes' lag
-__device__ __forceinline__ int32_t wv_period(int32_t QW, int32_t gw) { return max(QW, gw + 1); }
+// Iterations from a wave's pass to its next one: its words, or the lag of the
+// lanes.  On four waves (gw 256) each wave runs 65 iterations behind the one
+// above, and the first wave's next pass waits for the last wave: with a shorter
+// period it would wait before its own lanes have fed the waves between.
+constexpr int32_t WV_COOP_PERIOD = 4 * 65;
+__device__ __forceinline__ int32_t wv_period(int32_t QW, int32_t gw) { return max(QW, gw == 256 ? WV_COOP_PERIOD : gw + 1); }
 __device__ __forceinline__ uint32_t *wv_tile(const G2Dev &d, uint2 at, int32_t QW, int32_t strip, int32_t word, int32_t what) {
-    const int32_t lg = (int32_t)(at.y >> 8), gw = 1 << lg, u = strip >> 1, l = u & (gw - 1);
-    const uint32_t it = at.x + (uint32_t)((u >> lg) * wv_period(QW, gw) + word + l);
+    const bool coop = (at.y >> 8 & 15u) == 8u;
+    const int32_t lg = coop ? 6 : (int32_t)(at.y >> 8 & 15u), gw = 1 << lg, u = strip >> 1, l = u & (gw - 1);
+    const int32_t pass = u >> lg, own = coop ? pass >> 2 : pass;
+    const uint32_t it = at.x + (uint32_t)(own * wv_period(QW, coop ? 256 : gw) + word + l) + (coop ? (uint32_t)(pass & 3) * (at.y >> 12) : 0u);
     return d.tb + (size_t)it * WV_ITER + (uint32_t)(what + (strip & 1)) * WV_STREAM + ((at.y & 255u) + (uint32_t)l) * 8u;
 }
 

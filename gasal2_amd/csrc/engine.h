@@ -88,8 +88,8 @@ struct G2Dev {
     // ranked with their row (LOCAL: H <= 8191), 2: H alone.  When the census
     // refuses the score tables the lane kernels run the batch instead.
     uint32_t wave, wave_coop, wave64;
-    // WITH_TB on that path (wavetb.hip): the first wave64 sorted slots on 64
-    // lanes, the next wave16 (a multiple of four, or to the end) on 16, the rest
+    // WITH_TB on that path (wavetb.hip): after wave_coop and wave64 as above, the
+    // next wave16 slots (a multiple of four, or to the end) on 16 lanes, the rest
     // on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
     // and wv_strip (second best) max_tw words a slot, one per strip.
     uint32_t wave16;

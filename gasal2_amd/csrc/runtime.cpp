@@ -1008,22 +1008,29 @@ bool wave_tb_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw
     return g2_wave_fits(plain, sc, qw, tw, fast) == 1;
 }
 
-// Iterations of a pair on gw lanes of that path.
+// Iterations of a pair on gw lanes of that path; 256: of each of a block's four
+// waves, in whose region a pass in four falls.
 uint64_t wave_tb_iters(uint32_t qw, uint32_t tw, uint32_t gw) {
+    if (gw == 256) return (uint64_t)((tw + 511) / 512) * std::max(qw, 260u) + 64;   // WV_COOP_PERIOD
     return (uint64_t)((tw + 2 * gw - 1) / (2 * gw)) * std::max(qw, gw + 1) + gw;
 }
 
 // Lanes of a pair: 4 unless its iterations there would outlast the batch's
-// share of a SIMD (work: wave-iterations of the batch on 4 lanes; 1.5: a wave
-// alone on a SIMD against its share of a full one), else the least of 16 and
-// 64 that would not, else what is fewest iterations.
+// share of a SIMD (work: wave-iterations of the batch on 4 lanes; 3: a wave is one
+// of about three that share a SIMD, and the longest do not all start first), else the least of 16, 64
+// and 256 (from two passes of 64 lanes up; each wave starts 65 iterations after
+// the one above) that would not, else what is fewest iterations.  50,000 pairs of
+// 50-5000 bases LOCAL, DP: without the 256 13.6 ms, with it 9.4 (11.7 with 1.5 in
+// place of the 3, 10.1 with 6).
 uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double work) {
-    const double share = work / (g2_cu_count() * 4.0 + 1.0) / 1.5;
+    const double share = work / (g2_cu_count() * 4.0 + 1.0) / 3.0;
     uint32_t best = 4;
-    for (uint32_t gw : {4u, 16u, 64u}) {
-        const uint64_t its = wave_tb_iters(qw, tw, gw);
+    uint64_t least = ~0ull;
+    for (uint32_t gw : {4u, 16u, 64u, 256u}) {
+        if (gw == 256 && tw <= 128) break;
+        const uint64_t its = wave_tb_iters(qw, tw, gw) + (gw == 256 ? 195 : 0);
         if ((double)its <= share) return gw;
-        if (its < wave_tb_iters(qw, tw, best)) best = gw;
+        if (its < least) { least = its; best = gw; }
     }
     return best;
 }
@@ -1425,7 +1432,7 @@ G2Opts opts_of(const Parameters *p, const gasal_gpu_storage_t *s) {
     return o;
 }
 
-// The packed one-wave traceback path's launch (d.wave64, d.wave16) and the most
+// The packed one-wave traceback path's launch (d.wave_coop, 64, 16) and the most
 // iterations its waves can claim together: the batch's shapes in the device's
 // sorted order (k_keys), each bucket at its largest shape, every wave at its
 // longest pair's.
@@ -1454,13 +1461,16 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
     auto t_of = [&](uint32_t key) { return std::min(shape8_edge(key & 255u), tw); };
     double work = 0;
     for (const auto &r : runs) work += (double)r.second * wave_tb_iters(q_of(r.first), t_of(r.first), 4) / 16.0;
-    uint32_t n64 = 0, n16 = 0;
+    uint32_t n256 = 0, n64 = 0, n16 = 0;
+    const bool coop = wave_tb_iters(qw, tw, 256) < 1u << 20;   // a region's size is kept in 20 bits
     for (const auto &r : runs) {
         const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), work);
-        if (lanes == 64) n64 += r.second;
+        if (lanes == 256 && coop) n256 += r.second;
+        else if (lanes >= 64) n64 += r.second;
         if (lanes == 16) n16 += r.second;
     }
-    n16 = std::min((n16 + 3) & ~3u, n - n64);
+    n16 = std::min((n16 + 3) & ~3u, n - n256 - n64);
+    d.wave_coop = n256;
     d.wave64 = n64;
     d.wave16 = n16;
     uint64_t total = 0, longest = 0;
@@ -1472,10 +1482,10 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
             if (!room) {
                 total += longest;
                 longest = 0;
-                room = slot < n64 ? 1 : (slot < n64 + n16 ? 4 : 16);
+                room = slot < n256 + n64 ? 1 : (slot < n256 + n64 + n16 ? 4 : 16);
             }
-            const uint32_t g = slot < n64 ? 64 : (slot < n64 + n16 ? 16 : 4);
-            if (g != gw) its = wave_tb_iters(q_of(r.first), t_of(r.first), gw = g);
+            const uint32_t g = slot < n256 ? 256 : (slot < n256 + n64 ? 64 : (slot < n256 + n64 + n16 ? 16 : 4));
+            if (g != gw) its = wave_tb_iters(q_of(r.first), t_of(r.first), gw = g) * (g == 256 ? 4 : 1);
             longest = std::max(longest, its);
             const uint32_t take = std::min(c, room);
             c -= take;

@@ -18,7 +18,8 @@
 // enough, 16 and 64 for few or long ones.  Counters on 300,000 pairs of 100-300 x
 // 100-400 bases: 2.6 G wave instructions, VALU issue 65% of 7.1 ms, 18.7 GB
 // written.  100,000 pairs GLOBAL: 5.95 ms (one lane a pair, direction words) ->
-// 2.3; 50,000 pairs of 50-5000 bases LOCAL 32 -> 13.6; 50,000 pairs with second
+// 2.3; 50,000 pairs of 50-5000 bases LOCAL 32 -> 9.4 (13.6
+// with the longest on one wave); 50,000 pairs with second
 // best (half a wave a SIMD on two pairs a lane) 5.5 -> 1.6.
 //
 // The values are those of the lane kernels (k_local_fast, k_global), whose
@@ -48,10 +49,22 @@ __device__ __forceinline__ void rec_load(const uint32_t *p, uint32_t *w) {
     w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
 }
 
-// The pairs of one wave: slots slot0, slot0 + 1, ... below slot_end, GW lanes each.
-template <int MODE, bool SECOND, int GW>
-__device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, const uint32_t *lut16, uint32_t slot0,
-                                         uint32_t slot_end) {
+constexpr int WV_WAVES = 4;   // per block
+struct WvShared {
+    uint32_t lut16[16];          // score tables of the 16 target nibbles
+    uint32_t it0;                // COOP: the pair's first iteration
+    int32_t done[WV_WAVES];      // COOP: iterations whose records each wave has stored
+    int32_t end[WV_WAVES][4];    // COOP: each wave's best
+};
+
+// The pairs of one wave: slots slot0, slot0 + 1, ... below slot_end, GW lanes
+// each.  COOP: the block's four waves share one pair, wave w its passes w, w + 4,
+// ...; a pass follows the one above it by the iterations that one has stored.
+template <int MODE, bool SECOND, int GW, bool COOP>
+__device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvShared &sh, uint32_t slot0, uint32_t slot_end) {
+    const uint32_t *lut16 = sh.lut16;
+    constexpr int NW = COOP ? WV_WAVES : 1;
+    const int32_t wv = COOP ? (int32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) : 0;
     const int32_t lane = (int32_t)(threadIdx.x & (WAVE - 1)), l = lane & (GW - 1);
     const int32_t gapo = c.gapo, gape = c.gape;
     const pk16x2 gapoe2 = {(short)c.gapoe, (short)c.gapoe}, gape2 = {(short)c.gape, (short)c.gape};
@@ -62,15 +75,36 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
     const int32_t qlen = (int32_t)d.qlen[pr], tlen = (int32_t)d.tlen[pr];
     const int32_t QW = dregs((uint32_t)qlen), TW = dregs((uint32_t)tlen);   // at least one word each (the host checks)
     const uint32_t *Q = d.pq + (d.qoff[pr] >> 3), *T = d.pt + (d.toff[pr] >> 3);
-    const int32_t P = wv_period(QW, GW), npass = ok ? (TW + 2 * GW - 1) / (2 * GW) : 0, strips = ok ? TW : 0;
+    const int32_t passes = ok ? (TW + 2 * GW - 1) / (2 * GW) : 0;        // of the pair
+    const int32_t P = wv_period(QW, COOP ? 256 : GW), npass = (passes - wv + NW - 1) / NW, strips = ok ? TW : 0;   // npass: this wave's
     const int32_t its = wave_max<GW>(npass > 0 ? npass * P + GW : 0);
+    const int32_t log = COOP ? (passes + NW - 1) / NW * P + GW : its;    // iterations of a wave's region
     const bool slack = !__any(P < GW + 3);
     uint32_t it0 = 0;
-    if (lane == 0) it0 = atomicAdd(&d.aux[4], (uint32_t)its);
+    if (lane == 0 && wv == 0) it0 = atomicAdd(&d.aux[4], (uint32_t)(NW * log));
     it0 = __builtin_amdgcn_readfirstlane(it0);
-    uint32_t *out = d.tb + (size_t)it0 * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
-    if (ok && l == 0)
-        d.wv_at[pr] = make_uint2(it0, (uint32_t)lane | (uint32_t)(GW == 64 ? 6 : (GW == 16 ? 4 : 2)) << 8);
+    if (COOP) {
+        if (threadIdx.x == 0) sh.it0 = it0;
+        if (lane == 0) sh.done[wv] = 0;
+        __syncthreads();
+        it0 = __builtin_amdgcn_readfirstlane(sh.it0);
+    }
+    uint32_t *out = d.tb + (size_t)(it0 + (uint32_t)(wv * log)) * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
+    if (ok && l == 0 && wv == 0)
+        d.wv_at[pr] = make_uint2(it0, (uint32_t)lane | (uint32_t)(COOP ? 8 : (GW == 64 ? 6 : (GW == 16 ? 4 : 2))) << 8 |
+                                          (COOP ? (uint32_t)log << 12 : 0u));
+    auto strip_of = [&](int32_t k) -> int32_t { return 2 * (GW * (NW * k + wv) + l); };   // the lane's low strip of pass k
+    // COOP: the row above word j of the wave's pass k, from the wave of the pass
+    // above; waits until it is stored
+    const int32_t up = (wv + NW - 1) % NW;
+    auto coop_row = [&](int32_t k, int32_t j) -> const uint32_t * {
+        const int32_t it = (wv > 0 ? k : k - 1) * P + j + GW - 1;
+        const int32_t need = __builtin_amdgcn_readfirstlane(it + 2);   // the first lane's word; its record is stored an iteration later
+        const bool waits = __builtin_amdgcn_readfirstlane(NW * k + wv > 0 && k < npass && j < QW);
+        while (waits && __hip_atomic_load(&sh.done[up], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need)
+            __builtin_amdgcn_s_sleep(1);
+        return d.tb + (size_t)(it0 + (uint32_t)(up * log + it)) * WV_ITER + 3 * WV_STREAM + (GW - 1) * 8;
+    };
     auto hl = [&](int32_t R) -> int32_t { return R == 0 ? 0 : -(gapo + gape * R); };   // src/kernels/global.h:67-71
     // GLOBAL: H(column - 1) and E of the row above the matrix (src/kernels/global.h:57-60)
     auto top_row = [&](int32_t col) -> uint32_t {
@@ -79,11 +113,12 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
 
     // the lane's word and pass; before its first word it waits at the end of pass -1
     int32_t j = P - 1 - l, k = -1, sH = 0x7FFFFFFF;
-    uint32_t gL = T[min(2 * l, TW - 1)], gH = T[min(2 * l + 1, TW - 1)];   // target words of the next strips
+    uint32_t gL = T[min(strip_of(0), TW - 1)], gH = T[min(strip_of(0) + 1, TW - 1)];   // target words of the next strips
     uint32_t qcur = 0, qn = Q[0];                   // query word; the first lane's next one
     uint32_t row[8];                                // first lane: the row above, H one column back | E << 16
 #pragma unroll
     for (int kk = 0; kk < 8; kk++) row[kk] = top_row(kk);
+    if (COOP && wv > 0 && npass > 0) rec_load(coop_row(0, 0), row);
     uint32_t lutL[9], lutH[9], oH[8], carry = 0, qlast = 0;
     pk16x2 h[9], f[9], hb = zero2;                  // hb: bottom row's H one column back
 #pragma unroll
@@ -105,13 +140,13 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
         j++;
         const bool ended = j == QW && k >= 0, wrap = j == P;
         if (ended) {
-            const int32_t sL = 2 * (GW * k + l);
+            const int32_t sL = strip_of(k);
             if (sL < strips) strip_done(sL, best2 & 0xFFFFu, (int32_t)(bpos2 & 0xFFFFu), low2 & 0xFFFFu);
         }
         if (wrap) {   // the low strip of the next pass
             j = 0;
             k++;
-            const int32_t sL = 2 * (GW * k + l);
+            const int32_t sL = strip_of(k);
 #pragma unroll
             for (int m = 1; m < 9; m++) {
                 lutL[m] = lut16[(gL >> (32 - 4 * m)) & 15u];
@@ -122,14 +157,14 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
             best2 &= 0xFFFF0000u;
             low2 &= 0xFFFF0000u;
             col2 &= 0xFFFF0000u;
-            gL = T[min(sL + 2 * GW, TW - 1)];
+            gL = T[min(sL + 2 * GW * NW, TW - 1)];
         }
         qcur = from_above<GW>(qn, qcur);
         const uint32_t qodd = qcur & 0x07070707u, qeven = qcur & 0x70707070u;   // classes, neighbours cleared
         // the first lane's next word
         const int32_t jn = j + 1 == P ? 0 : j + 1, kn = j + 1 == P ? k + 1 : k;
-        const bool next_row = l == 0 && kn > 0 && kn < npass && jn < QW;
-        const uint32_t *above = out + (ptrdiff_t)(GW - P) * (ptrdiff_t)WV_ITER + 3 * WV_STREAM + (GW - 1) * 8;
+        const bool next_row = l == 0 && NW * kn + wv > 0 && kn < npass && jn < QW;
+        const uint32_t *above = out + (ptrdiff_t)(GW - P) * (ptrdiff_t)WV_ITER + 3 * WV_STREAM + (GW - 1) * 8;   // !COOP
         if (l == 0) qn = Q[min(jn, QW - 1)];
         uint32_t w[8];
 #pragma unroll
@@ -177,7 +212,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
                 if (it > 0) rec_store(out - WV_ITER + 3 * WV_STREAM, oH);
                 if (ended && sH < strips) strip_done(sH, best2 >> 16, (int32_t)(bpos2 >> 16), low2 >> 16);
                 if (wrap) {   // and its strip of the next pass, from the next step on
-                    sH = 2 * (GW * k + l) + 1;
+                    sH = strip_of(k) + 1;
 #pragma unroll
                     for (int m = 1; m < 9; m++) {
                         lutH[m] = lut16[(gH >> (32 - 4 * m)) & 15u];
@@ -188,7 +223,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
                     best2 &= 0xFFFFu;
                     low2 &= 0xFFFFu;
                     col2 &= 0xFFFFu;
-                    gH = T[min(sH + 2 * GW, TW - 1)];
+                    gH = T[min(sH + 2 * GW * NW, TW - 1)];
                 }
                 uint32_t v[8];
 #pragma unroll
@@ -200,7 +235,10 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
                 // ago by the last lane: two and more, and all but the newest
                 // eight of the wave's accesses hold it (an iteration issues
                 // eight stores and more).
-                if (kk == 3) {
+                if (COOP && kk == 3) {
+                    __hip_atomic_store(&sh.done[wv], it + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    above = coop_row(kn, jn);
+                } else if (kk == 3) {
                     if (slack) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
                     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 }
@@ -210,7 +248,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
                     row[o] = a.x; row[o + 1] = a.y; row[o + 2] = a.z; row[o + 3] = a.w;
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) row[o + i] = kn == 0 ? top_row(8 * jn + o + i) : 0u;
+                    for (int i = 0; i < 4; i++) row[o + i] = NW * kn + wv == 0 ? top_row(8 * jn + o + i) : 0u;
                 }
             }
         }
@@ -218,8 +256,9 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
     }
 
     if (MODE == TB_GLOBAL) {   // the score: row tlen, column qlen of the last tile, rebuilt (src/kernels/global.h:98-103, 299)
+        if (COOP) __syncthreads();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-        if (!ok || l != 0) return;
+        if (!ok || l != 0 || wv != 0) return;
         const uint2 at = d.wv_at[pr];
         uint32_t top[8], left[8];
         rec_load(wv_tile(d, at, QW, TW - 1, QW - 1, WV_LEFT), left);
@@ -254,26 +293,43 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, cons
         const int32_t ov = __shfl_xor(bv, off), os = __shfl_xor(bs, off), oc = __shfl_xor(bc, off), orow = __shfl_xor(br, off);
         if (ov > bv || (ov == bv && (os < bs || (os == bs && oc < bc)))) { bv = ov; bs = os; bc = oc; br = orow; }
     }
-    if (ok && l == 0) {
+    if (COOP) {   // and the block's waves in the same way
+        if (lane == 0) { sh.end[wv][0] = bv; sh.end[wv][1] = bs; sh.end[wv][2] = bc; sh.end[wv][3] = br; }
+        __syncthreads();
+        for (int w = 0; w < NW; w++) {
+            const int32_t *o = sh.end[w];
+            if (o[0] > bv || (o[0] == bv && (o[1] < bs || (o[1] == bs && o[2] < bc)))) { bv = o[0]; bs = o[1]; bc = o[2]; br = o[3]; }
+        }
+    }
+    if (ok && l == 0 && wv == 0) {
         d.score[pr] = bv;
         d.qend[pr] = bv > 0 ? bc : 0;
         d.tend[pr] = bv > 0 ? bs * 8 + br : 0;
     }
 }
 
+// Launch: a block for each of the first d.wave_coop sorted slots, then a wave for
+// each of the next d.wave64, for four of the next d.wave16 and for sixteen of the
+// others, four waves a block.
 template <int MODE, bool SECOND>
-__global__ __launch_bounds__(WAVE) void k_wave_tb(G2Dev d, G2Scores c) {
+__global__ __launch_bounds__(WV_WAVES * WAVE) void k_wave_tb(G2Dev d, G2Scores c) {
     const uint32_t census = d.aux[0];
     if (!census_fast(census)) return;   // the lane kernels take this batch
-    __shared__ uint32_t lut16[16];
+    __shared__ WvShared sh;
     if (threadIdx.x < 16)
-        lut16[threadIdx.x] = MODE == TB_GLOBAL ? score_lut<true>(c, 0, census, threadIdx.x)
-                                               : score_lut(c, c.has_np ? -c.np : 0, census, threadIdx.x);
+        sh.lut16[threadIdx.x] = MODE == TB_GLOBAL ? score_lut<true>(c, 0, census, threadIdx.x)
+                                                  : score_lut(c, c.has_np ? -c.np : 0, census, threadIdx.x);
     __syncthreads();
-    const uint32_t b = blockIdx.x, b1 = d.wave64, b2 = b1 + (d.wave16 + 3) / 4, s1 = d.wave64, s2 = s1 + d.wave16;
-    if (b < b1) wv_pairs<MODE, SECOND, 64>(d, c, lut16, b, s1);
-    else if (b < b2) wv_pairs<MODE, SECOND, 16>(d, c, lut16, s1 + 4 * (b - b1), s2);
-    else wv_pairs<MODE, SECOND, 4>(d, c, lut16, s2 + 16 * (b - b2), d.n);
+    const uint32_t b = blockIdx.x, s0 = d.wave_coop, s1 = s0 + d.wave64, s2 = s1 + d.wave16;
+    if (b < s0) {
+        wv_pairs<MODE, SECOND, 64, true>(d, c, sh, b, s0);
+        return;
+    }
+    const uint32_t u = WV_WAVES * (b - s0) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t u1 = d.wave64, u2 = u1 + (d.wave16 + 3) / 4, u3 = u2 + (d.n - s2 + 15) / 16;
+    if (u < u1) wv_pairs<MODE, SECOND, 64, false>(d, c, sh, s0 + u, s1);
+    else if (u < u2) wv_pairs<MODE, SECOND, 16, false>(d, c, sh, s1 + 4 * (u - u1), s2);
+    else if (u < u3) wv_pairs<MODE, SECOND, 4, false>(d, c, sh, s2 + 16 * (u - u2), d.n);
 }
 
 // Second best from the strips' records (the header's rule).  A strip's record:
@@ -609,17 +665,18 @@ __global__ __launch_bounds__(WAVE) void k_wave_walk(G2Dev d, G2Scores c) {
 }  // namespace
 
 hipError_t g2_wave_tb_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t s) {
-    const uint32_t blocks = d.wave64 + (d.wave16 + 3) / 4 + (d.n - d.wave64 - d.wave16 + 15) / 16;
+    const uint32_t waves4 = d.wave64 + (d.wave16 + 3) / 4 + (d.n - d.wave_coop - d.wave64 - d.wave16 + 15) / 16;
+    const uint32_t blocks = d.wave_coop + (waves4 + WV_WAVES - 1) / WV_WAVES;
     if (op.algo == A_GLOBAL) {
-        k_wave_tb<TB_GLOBAL, false><<<blocks, WAVE, 0, s>>>(d, sc);
+        k_wave_tb<TB_GLOBAL, false><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
     } else if (op.second) {
-        k_wave_tb<TB_LOCAL, true><<<blocks, WAVE, 0, s>>>(d, sc);
+        k_wave_tb<TB_LOCAL, true><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
         const uint32_t waves = (d.n + WAVE - 1) / WAVE;
         k_second_scan<<<waves, WAVE, 0, s>>>(d);
         k_second_strips<<<waves < 4096 ? waves : 4096, WAVE, 0, s>>>(d, sc);
         k_second_out<<<(d.n + 255) / 256, 256, 0, s>>>(d);
     } else {
-        k_wave_tb<TB_LOCAL, false><<<blocks, WAVE, 0, s>>>(d, sc);
+        k_wave_tb<TB_LOCAL, false><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
     }
     return hipGetLastError();
 }

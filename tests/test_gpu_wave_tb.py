@@ -94,3 +94,20 @@ def test_no_score_tables(algo, second):
     q = bytearray(b.query(3))
     q[5:7] = b"IA"
     both_paths(g.make_batch([bytes(q)] + [b.query(i) for i in range(1, b.n)], [b.target(i) for i in range(b.n)]), algo, second)
+
+
+@pytest.mark.parametrize("algo,second", MODES)
+def test_long_pairs_on_four_waves(algo, second):
+    """Targets of 2 to 9 passes of 128 strips, the block's waves with unlike numbers of them."""
+    rng = np.random.default_rng(4700)
+    qs, ts = [], []
+    for lq, lt in ((2000, 2048), (2000, 2049), (1500, 4096), (1500, 4097), (3000, 5200), (900, 9100), (4000, 3100), (40, 4200)):
+        t = rng.choice(list(b"ACGT"), lt).astype(np.uint8)
+        q = rng.choice(list(b"ACGT"), lq).astype(np.uint8)
+        m, o = min(lq, lt), max(lt - lq, 0) // 2
+        q[:m] = t[o:o + m]
+        q[rng.random(lq) < 0.08] = ord("G")
+        q = np.delete(q, range(lq // 2, lq // 2 + 9))
+        qs.append(q.tobytes())
+        ts.append(t.tobytes())
+    both_paths(g.make_batch(qs, ts), algo, second)
