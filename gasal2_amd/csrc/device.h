@@ -78,9 +78,9 @@ __device__ __forceinline__ pk16x2 prank(pk16x2 h, uint32_t r2) {
 // the previous lane's v within the group; the group's first lane: first
 template <int GW>
 __device__ __forceinline__ uint32_t from_above(uint32_t first, uint32_t v) {
-    static_assert(GW == 4 || GW == 16 || GW == 64, "lanes of a group");
-    const uint32_t w = (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, GW == 64 ? 0x138 : 0x111, 0xF, 0xF, false);
-    return GW == 4 && (threadIdx.x & 3u) == 0 ? first : w;
+    static_assert(GW == 4 || GW == 16 || GW == 32 || GW == 64, "lanes of a group");
+    const uint32_t w = (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, GW >= 32 ? 0x138 : 0x111, 0xF, 0xF, false);
+    return (GW == 4 || GW == 32) && (threadIdx.x & (GW - 1u)) == 0 ? first : w;
 }
 // maximum over the wave of a value that is uniform within groups of GW lanes
 template <int GW = 16>

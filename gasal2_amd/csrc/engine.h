@@ -89,10 +89,10 @@ struct G2Dev {
     // refuses the score tables the lane kernels run the batch instead.
     uint32_t wave, wave_coop, wave64;
     // WITH_TB on that path (wavetb.hip): after wave_coop and wave64 as above, the
-    // next wave16 slots (a multiple of four, or to the end) on 16 lanes, the rest
-    // on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
+    // next wave32 and wave16 slots (whole waves of them, or to the end) on 32 and
+    // 16 lanes, the rest on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
     // and wv_strip (second best) max_tw words a slot, one per strip.
-    uint32_t wave16;
+    uint32_t wave32, wave16;
     uint2 *wv_at;
     uint32_t *wv_strip;
     uint2 *wv_item;                  // second best: strips to recompute (k_second_strips), at most one per strip

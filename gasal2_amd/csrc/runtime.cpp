@@ -1015,22 +1015,29 @@ uint64_t wave_tb_iters(uint32_t qw, uint32_t tw, uint32_t gw) {
     return (uint64_t)((tw + 2 * gw - 1) / (2 * gw)) * std::max(qw, gw + 1) + gw;
 }
 
-// Lanes of a pair: 4 unless its iterations there would outlast the batch's
-// share of a SIMD (work: wave-iterations of the batch on 4 lanes; 3: a wave is one
-// of about three that share a SIMD, and the longest do not all start first), else the least of 16, 64
-// and 256 (from two passes of 64 lanes up; each wave starts 65 iterations after
-// the one above) that would not, else what is fewest iterations.  50,000 pairs of
-// 50-5000 bases LOCAL, DP: without the 256 13.6 ms, with it 9.4 (11.7 with 1.5 in
-// place of the 3, 10.1 with 6).
-uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double work) {
-    const double share = work / (g2_cu_count() * 4.0 + 1.0) / 3.0;
+// Lanes of a pair.  load: iterations a SIMD runs when the batch's work is on 4
+// lanes.  The fewest lanes on which the pair's own iterations do not outlast the
+// batch (load / 3: a wave is one of about three that share a SIMD; on 4 lanes load
+// / 1.5 where the longest pair's iterations there are at most four times the
+// load, since such a batch's waves all start together, while after long pairs the
+// 4-lane waves start last); if none, those for which the pair's time alone
+// and the batch's, were all its pairs alike, are together least (a wave alone on
+// a SIMD takes 2.5 us an iteration, a full SIMD 1.15 us for each).  256: a
+// block's four waves, from two passes of 64 lanes up, each 65 iterations behind
+// the one above.  50,000 pairs of 50-5000 bases LOCAL, DP: without the 256 13.6
+// ms, with it 9.2 (10.7 with load / 1.5 on 4 lanes, 10.1 with load / 6); 64 pairs
+// of 100-300 bases on 16 lanes 248 us, on 32 205; 45,000 with second best 1.44 ms
+// with load / 1.5, 1.71 with load / 3.
+uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double load, double longest4) {
+    const double own4 = 4.0 * wave_tb_iters(qw, tw, 4);
     uint32_t best = 4;
-    uint64_t least = ~0ull;
-    for (uint32_t gw : {4u, 16u, 64u, 256u}) {
+    double least = 1e300;
+    for (uint32_t gw : {4u, 16u, 32u, 64u, 256u}) {
         if (gw == 256 && tw <= 128) break;
-        const uint64_t its = wave_tb_iters(qw, tw, gw) + (gw == 256 ? 195 : 0);
-        if ((double)its <= share) return gw;
-        if (its < least) { least = its; best = gw; }
+        const double its = (double)wave_tb_iters(qw, tw, gw) + (gw == 256 ? 195 : 0);
+        if (its <= load / (gw == 4 && longest4 <= 4.0 * load ? 1.5 : 3.0)) return gw;
+        const double cost = 2.5 * its + 1.15 * load * its * gw / own4;
+        if (cost < least) { least = cost; best = gw; }
     }
     return best;
 }
@@ -1452,28 +1459,47 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
             runs.back().second++;
         }
     } else {
-        m->h_khist.assign(G2_SHAPE_BUCKETS, 0u);
-        for (uint32_t k = 0; k < n; k++) m->h_khist[key_of(k)]++;
-        for (uint32_t key = G2_SHAPE_BUCKETS; key-- > 0;)
-            if (m->h_khist[key]) runs.push_back({key, m->h_khist[key]});
+        // counters stay zero between batches; only rows that hold pairs are read
+        m->h_khist.resize(G2_SHAPE_BUCKETS, 0u);
+        bool rows[G2_SHAPE_ROWS] = {};
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t key = key_of(k);
+            m->h_khist[key]++;
+            rows[key >> 8] = true;
+        }
+        for (uint32_t row = G2_SHAPE_ROWS; row-- > 0;)
+            for (uint32_t c = 256; rows[row] && c-- > 0;)
+                if (uint32_t &v = m->h_khist[row * 256 + c]) {
+                    runs.push_back({row * 256 + c, v});
+                    v = 0;
+                }
     }
     auto q_of = [&](uint32_t key) { return std::min(shape8_edge((key >> 8) & 255u), qw); };
     auto t_of = [&](uint32_t key) { return std::min(shape8_edge(key & 255u), tw); };
-    double work = 0;
-    for (const auto &r : runs) work += (double)r.second * wave_tb_iters(q_of(r.first), t_of(r.first), 4) / 16.0;
-    uint32_t n256 = 0, n64 = 0, n16 = 0;
+    double work = 0, longest4 = 0;
+    for (const auto &r : runs) {
+        const double its = (double)wave_tb_iters(q_of(r.first), t_of(r.first), 4);
+        work += r.second * its / 16.0;
+        longest4 = std::max(longest4, its);
+    }
+    const double load = work / (4.0 * std::max(g2_cu_count(), 1u));
+    uint32_t n256 = 0, n64 = 0, n32 = 0, n16 = 0;
     const bool coop = wave_tb_iters(qw, tw, 256) < 1u << 20;   // a region's size is kept in 20 bits
     for (const auto &r : runs) {
-        const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), work);
+        const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), load, longest4);
         if (lanes == 256 && coop) n256 += r.second;
         else if (lanes >= 64) n64 += r.second;
+        if (lanes == 32) n32 += r.second;
         if (lanes == 16) n16 += r.second;
     }
-    n16 = std::min((n16 + 3) & ~3u, n - n256 - n64);
+    n32 = std::min((n32 + 1) & ~1u, n - n256 - n64);
+    n16 = std::min((n16 + 3) & ~3u, n - n256 - n64 - n32);
     d.wave_coop = n256;
     d.wave64 = n64;
+    d.wave32 = n32;
     d.wave16 = n16;
     uint64_t total = 0, longest = 0;
+    const uint32_t s64 = n256 + n64, s32 = s64 + n32, s16 = s32 + n16;
     uint32_t slot = 0, room = 0;
     for (const auto &r : runs) {
         uint32_t c = r.second, gw = 0;
@@ -1482,9 +1508,9 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
             if (!room) {
                 total += longest;
                 longest = 0;
-                room = slot < n256 + n64 ? 1 : (slot < n256 + n64 + n16 ? 4 : 16);
+                room = slot < s64 ? 1 : (slot < s32 ? 2 : (slot < s16 ? 4 : 16));
             }
-            const uint32_t g = slot < n256 ? 256 : (slot < n256 + n64 ? 64 : (slot < n256 + n64 + n16 ? 16 : 4));
+            const uint32_t g = slot < n256 ? 256 : (slot < s64 ? 64 : (slot < s32 ? 32 : (slot < s16 ? 16 : 4)));
             if (g != gw) its = wave_tb_iters(q_of(r.first), t_of(r.first), gw = g) * (g == 256 ? 4 : 1);
             longest = std::max(longest, its);
             const uint32_t take = std::min(c, room);

@@ -1,4 +1,4 @@
-// wavetb.hip -- LOCAL and GLOBAL WITH_TB on groups of 4, 16 or 64 lanes per
+// wavetb.hip -- LOCAL and GLOBAL WITH_TB on groups of 4, 16, 32 or 64 lanes per
 // pair, with the checkpoints the traceback rebuilds its tiles from.
 //
 // Lane l of pass k holds target strips 2 (GW k + l) and the next one (8 rows
@@ -15,7 +15,7 @@
 // whole lines: a record a lane, 64 lanes side by side), times the share of lanes
 // and iterations that hold cells (a pair fills its lanes in GW iterations;
 // strips are rounded up to 2 GW).  Hence 4 lanes wherever the batch has pairs
-// enough, 16 and 64 for few or long ones.  Counters on 300,000 pairs of 100-300 x
+// enough, more for few or long ones.  Counters on 300,000 pairs of 100-300 x
 // 100-400 bases: 2.6 G wave instructions, VALU issue 65% of 7.1 ms, 18.7 GB
 // written.  100,000 pairs GLOBAL: 5.95 ms (one lane a pair, direction words) ->
 // 2.3; 50,000 pairs of 50-5000 bases LOCAL 32 -> 9.4 (13.6
@@ -91,7 +91,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
     }
     uint32_t *out = d.tb + (size_t)(it0 + (uint32_t)(wv * log)) * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
     if (ok && l == 0 && wv == 0)
-        d.wv_at[pr] = make_uint2(it0, (uint32_t)lane | (uint32_t)(COOP ? 8 : (GW == 64 ? 6 : (GW == 16 ? 4 : 2))) << 8 |
+        d.wv_at[pr] = make_uint2(it0, (uint32_t)lane | (uint32_t)(COOP ? 8 : __builtin_ctz(GW)) << 8 |
                                           (COOP ? (uint32_t)log << 12 : 0u));
     auto strip_of = [&](int32_t k) -> int32_t { return 2 * (GW * (NW * k + wv) + l); };   // the lane's low strip of pass k
     // COOP: the row above word j of the wave's pass k, from the wave of the pass
@@ -309,8 +309,8 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
 }
 
 // Launch: a block for each of the first d.wave_coop sorted slots, then a wave for
-// each of the next d.wave64, for four of the next d.wave16 and for sixteen of the
-// others, four waves a block.
+// each of the next d.wave64, for two of the next d.wave32, four of the next
+// d.wave16 and sixteen of the others, four waves a block.
 template <int MODE, bool SECOND>
 __global__ __launch_bounds__(WV_WAVES * WAVE) void k_wave_tb(G2Dev d, G2Scores c) {
     const uint32_t census = d.aux[0];
@@ -320,16 +320,17 @@ __global__ __launch_bounds__(WV_WAVES * WAVE) void k_wave_tb(G2Dev d, G2Scores c
         sh.lut16[threadIdx.x] = MODE == TB_GLOBAL ? score_lut<true>(c, 0, census, threadIdx.x)
                                                   : score_lut(c, c.has_np ? -c.np : 0, census, threadIdx.x);
     __syncthreads();
-    const uint32_t b = blockIdx.x, s0 = d.wave_coop, s1 = s0 + d.wave64, s2 = s1 + d.wave16;
+    const uint32_t b = blockIdx.x, s0 = d.wave_coop, s1 = s0 + d.wave64, s2 = s1 + d.wave32, s3 = s2 + d.wave16;
     if (b < s0) {
         wv_pairs<MODE, SECOND, 64, true>(d, c, sh, b, s0);
         return;
     }
     const uint32_t u = WV_WAVES * (b - s0) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t u1 = d.wave64, u2 = u1 + (d.wave16 + 3) / 4, u3 = u2 + (d.n - s2 + 15) / 16;
+    const uint32_t u1 = d.wave64, u2 = u1 + (d.wave32 + 1) / 2, u3 = u2 + (d.wave16 + 3) / 4, u4 = u3 + (d.n - s3 + 15) / 16;
     if (u < u1) wv_pairs<MODE, SECOND, 64, false>(d, c, sh, s0 + u, s1);
-    else if (u < u2) wv_pairs<MODE, SECOND, 16, false>(d, c, sh, s1 + 4 * (u - u1), s2);
-    else if (u < u3) wv_pairs<MODE, SECOND, 4, false>(d, c, sh, s2 + 16 * (u - u2), d.n);
+    else if (u < u2) wv_pairs<MODE, SECOND, 32, false>(d, c, sh, s1 + 2 * (u - u1), s2);
+    else if (u < u3) wv_pairs<MODE, SECOND, 16, false>(d, c, sh, s2 + 4 * (u - u2), s3);
+    else if (u < u4) wv_pairs<MODE, SECOND, 4, false>(d, c, sh, s3 + 16 * (u - u3), d.n);
 }
 
 // Second best from the strips' records (the header's rule).  A strip's record:
@@ -665,15 +666,16 @@ __global__ __launch_bounds__(WAVE) void k_wave_walk(G2Dev d, G2Scores c) {
 }  // namespace
 
 hipError_t g2_wave_tb_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t s) {
-    const uint32_t waves4 = d.wave64 + (d.wave16 + 3) / 4 + (d.n - d.wave_coop - d.wave64 - d.wave16 + 15) / 16;
-    const uint32_t blocks = d.wave_coop + (waves4 + WV_WAVES - 1) / WV_WAVES;
+    const uint32_t narrow = d.n - d.wave_coop - d.wave64 - d.wave32 - d.wave16;
+    const uint32_t waves = d.wave64 + (d.wave32 + 1) / 2 + (d.wave16 + 3) / 4 + (narrow + 15) / 16;
+    const uint32_t blocks = d.wave_coop + (waves + WV_WAVES - 1) / WV_WAVES;
     if (op.algo == A_GLOBAL) {
         k_wave_tb<TB_GLOBAL, false><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
     } else if (op.second) {
         k_wave_tb<TB_LOCAL, true><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
-        const uint32_t waves = (d.n + WAVE - 1) / WAVE;
-        k_second_scan<<<waves, WAVE, 0, s>>>(d);
-        k_second_strips<<<waves < 4096 ? waves : 4096, WAVE, 0, s>>>(d, sc);
+        const uint32_t groups = (d.n + WAVE - 1) / WAVE;
+        k_second_scan<<<groups, WAVE, 0, s>>>(d);
+        k_second_strips<<<groups < 4096 ? groups : 4096, WAVE, 0, s>>>(d, sc);
         k_second_out<<<(d.n + 255) / 256, 256, 0, s>>>(d);
     } else {
         k_wave_tb<TB_LOCAL, false><<<blocks, WV_WAVES * WAVE, 0, s>>>(d, sc);
