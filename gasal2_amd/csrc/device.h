@@ -179,8 +179,8 @@ __device__ __forceinline__ void ck_tile(const uint32_t *top, const uint32_t *lef
 // lane -- left column state of the low and the high strip, bottom row of the
 // low and the high strip -- so that every store of a wave covers whole lines.
 // at: the pair's first iteration, first lane | log2(lanes of its group) << 8; for
-// a pair on a block's four waves 8 there, | iterations of a wave's region << 12
-// (the four regions follow each other, passes dealt to them in turn).
+// a pair on a block's four waves 8 there, | its passes << 12 (dealt to the waves in
+// turn; the waves' regions follow each other).
 constexpr uint32_t WV_STREAM = WAVE * 8, WV_ITER = 4 * WV_STREAM;   // dwords
 enum { WV_LEFT = 0, WV_BOTTOM = 2 };
 // Iterations from a wave's pass to its next one: its words, or the lag of the
@@ -189,11 +189,16 @@ enum { WV_LEFT = 0, WV_BOTTOM = 2 };
 // period it would wait before its own lanes have fed the waves between.
 constexpr int32_t WV_COOP_PERIOD = 4 * 65;
 __device__ __forceinline__ int32_t wv_period(int32_t QW, int32_t gw) { return max(QW, gw == 256 ? WV_COOP_PERIOD : gw + 1); }
+// first iteration of wave w's region among those of a pair on four waves
+__device__ __forceinline__ uint32_t wv_region(uint32_t passes, int32_t P, uint32_t w) {
+    return w * WAVE + (uint32_t)P * (w * (passes >> 2) + min(w, passes & 3u));
+}
 __device__ __forceinline__ uint32_t *wv_tile(const G2Dev &d, uint2 at, int32_t QW, int32_t strip, int32_t word, int32_t what) {
     const bool coop = (at.y >> 8 & 15u) == 8u;
     const int32_t lg = coop ? 6 : (int32_t)(at.y >> 8 & 15u), gw = 1 << lg, u = strip >> 1, l = u & (gw - 1);
     const int32_t pass = u >> lg, own = coop ? pass >> 2 : pass;
-    const uint32_t it = at.x + (uint32_t)(own * wv_period(QW, coop ? 256 : gw) + word + l) + (coop ? (uint32_t)(pass & 3) * (at.y >> 12) : 0u);
+    const int32_t P = wv_period(QW, coop ? 256 : gw);
+    const uint32_t it = at.x + (uint32_t)(own * P + word + l) + (coop ? wv_region(at.y >> 12, P, (uint32_t)(pass & 3)) : 0u);
     return d.tb + (size_t)it * WV_ITER + (uint32_t)(what + (strip & 1)) * WV_STREAM + ((at.y & 255u) + (uint32_t)l) * 8u;
 }
 

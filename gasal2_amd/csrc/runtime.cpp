@@ -1008,8 +1008,8 @@ bool wave_tb_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw
     return g2_wave_fits(plain, sc, qw, tw, fast) == 1;
 }
 
-// Iterations of a pair on gw lanes of that path; 256: of each of a block's four
-// waves, in whose region a pass in four falls.
+// Iterations of a pair on gw lanes of that path; 256: of the first of a block's
+// four waves, which take the passes in turn.
 uint64_t wave_tb_iters(uint32_t qw, uint32_t tw, uint32_t gw) {
     if (gw == 256) return (uint64_t)((tw + 511) / 512) * std::max(qw, 260u) + 64;   // WV_COOP_PERIOD
     return (uint64_t)((tw + 2 * gw - 1) / (2 * gw)) * std::max(qw, gw + 1) + gw;
@@ -1404,7 +1404,7 @@ void ensure(T *&p, size_t &cap_bytes, size_t need_bytes) {
     if (p) G2_CHECK(hipFree(p));
     p = nullptr;
     cap_bytes = 0;
-    size_t b = need_bytes + need_bytes / 8 + 256;
+    size_t b = need_bytes + std::min<size_t>(need_bytes / 8, 1ull << 30) + 256;   // room to grow, at most 1 GiB of it
     hipError_t e = hipMalloc((void **)&p, b);
     if (e != hipSuccess) {
         p = nullptr;
@@ -1484,11 +1484,10 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
     }
     const double load = work / (4.0 * std::max(g2_cu_count(), 1u));
     uint32_t n256 = 0, n64 = 0, n32 = 0, n16 = 0;
-    const bool coop = wave_tb_iters(qw, tw, 256) < 1u << 20;   // a region's size is kept in 20 bits
     for (const auto &r : runs) {
         const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), load, longest4);
-        if (lanes == 256 && coop) n256 += r.second;
-        else if (lanes >= 64) n64 += r.second;
+        if (lanes == 256) n256 += r.second;
+        if (lanes == 64) n64 += r.second;
         if (lanes == 32) n32 += r.second;
         if (lanes == 16) n16 += r.second;
     }
@@ -1511,7 +1510,11 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
                 room = slot < s64 ? 1 : (slot < s32 ? 2 : (slot < s16 ? 4 : 16));
             }
             const uint32_t g = slot < n256 ? 256 : (slot < s64 ? 64 : (slot < s32 ? 32 : (slot < s16 ? 16 : 4)));
-            if (g != gw) its = wave_tb_iters(q_of(r.first), t_of(r.first), gw = g) * (g == 256 ? 4 : 1);
+            if (g != gw) {
+                gw = g;
+                const uint32_t kq = q_of(r.first), kt = t_of(r.first);
+                its = g == 256 ? (uint64_t)((kt + 127) / 128) * std::max(kq, 260u) + 256 : wave_tb_iters(kq, kt, g);
+            }
             longest = std::max(longest, its);
             const uint32_t take = std::min(c, room);
             c -= take;
@@ -1791,7 +1794,9 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         // storage's own tile buffer counted as free: it is reused), so that
         // several storages of a large batch fit beside each other; else
         // regions sized per group (about half the bytes on mixed lengths).
-        bool one = one_size <= g_tb_one_size_max;
+        // The packed one-wave path's fallback takes what that path's checkpoints
+        // take, or per-group regions.
+        bool one = one_size <= (wave_tb ? std::min(g_tb_one_size_max, wave_bytes - std::min(wave_bytes, wf_bytes)) : g_tb_one_size_max);
         if (one) {
             size_t free_b = 0, total_b = 0;
             if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)

@@ -78,10 +78,9 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
     const int32_t passes = ok ? (TW + 2 * GW - 1) / (2 * GW) : 0;        // of the pair
     const int32_t P = wv_period(QW, COOP ? 256 : GW), npass = (passes - wv + NW - 1) / NW, strips = ok ? TW : 0;   // npass: this wave's
     const int32_t its = wave_max<GW>(npass > 0 ? npass * P + GW : 0);
-    const int32_t log = COOP ? (passes + NW - 1) / NW * P + GW : its;    // iterations of a wave's region
     const bool slack = !__any(P < GW + 3);
     uint32_t it0 = 0;
-    if (lane == 0 && wv == 0) it0 = atomicAdd(&d.aux[4], (uint32_t)(NW * log));
+    if (lane == 0 && wv == 0) it0 = atomicAdd(&d.aux[4], COOP ? wv_region((uint32_t)passes, P, WV_WAVES) : (uint32_t)its);
     it0 = __builtin_amdgcn_readfirstlane(it0);
     if (COOP) {
         if (threadIdx.x == 0) sh.it0 = it0;
@@ -89,10 +88,10 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
         __syncthreads();
         it0 = __builtin_amdgcn_readfirstlane(sh.it0);
     }
-    uint32_t *out = d.tb + (size_t)(it0 + (uint32_t)(wv * log)) * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
+    uint32_t *out = d.tb + (size_t)(it0 + (COOP ? wv_region((uint32_t)passes, P, (uint32_t)wv) : 0u)) * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
     if (ok && l == 0 && wv == 0)
         d.wv_at[pr] = make_uint2(it0, (uint32_t)lane | (uint32_t)(COOP ? 8 : __builtin_ctz(GW)) << 8 |
-                                          (COOP ? (uint32_t)log << 12 : 0u));
+                                          (COOP ? (uint32_t)passes << 12 : 0u));
     auto strip_of = [&](int32_t k) -> int32_t { return 2 * (GW * (NW * k + wv) + l); };   // the lane's low strip of pass k
     // COOP: the row above word j of the wave's pass k, from the wave of the pass
     // above; waits until it is stored
@@ -103,7 +102,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
         const bool waits = __builtin_amdgcn_readfirstlane(NW * k + wv > 0 && k < npass && j < QW);
         while (waits && __hip_atomic_load(&sh.done[up], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need)
             __builtin_amdgcn_s_sleep(1);
-        return d.tb + (size_t)(it0 + (uint32_t)(up * log + it)) * WV_ITER + 3 * WV_STREAM + (GW - 1) * 8;
+        return d.tb + (size_t)(it0 + wv_region((uint32_t)passes, P, (uint32_t)up) + (uint32_t)it) * WV_ITER + 3 * WV_STREAM + (GW - 1) * 8;
     };
     auto hl = [&](int32_t R) -> int32_t { return R == 0 ? 0 : -(gapo + gape * R); };   // src/kernels/global.h:67-71
     // GLOBAL: H(column - 1) and E of the row above the matrix (src/kernels/global.h:57-60)
