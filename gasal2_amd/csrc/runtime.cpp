@@ -1404,7 +1404,7 @@ void ensure(T *&p, size_t &cap_bytes, size_t need_bytes) {
     if (p) G2_CHECK(hipFree(p));
     p = nullptr;
     cap_bytes = 0;
-    size_t b = need_bytes + std::min<size_t>(need_bytes / 8, 1ull << 30) + 256;   // room to grow, at most 1 GiB of it
+    size_t b = need_bytes + need_bytes / 8 + 256;
     hipError_t e = hipMalloc((void **)&p, b);
     if (e != hipSuccess) {
         p = nullptr;
@@ -1630,6 +1630,19 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // counted as free: it is reused): about 64 B per tile and 5 KB a pair.
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
+    if (wave_tb && op.algo == LOCAL && n > 65536 && g2_get_dispatch() == 0) {
+        // a large batch that the lane kernels clearly run faster is told by 4096
+        // of its pairs (a pass over 1M pairs took 2 ms of a 24.7 ms step)
+        uint64_t tiles = 0, work = 0;
+        const uint32_t step = n / 4096;
+        for (uint32_t k = 0; k < 4096; k++) {
+            const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
+            tiles += (uint64_t)kq * kt;
+            work += wave_tb_iters(kq, kt, 4);
+        }
+        const double scale = n / 4096.0;
+        wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, 0.75 * scale * work / 16.0);
+    }
     uint64_t wave_strips = 0, path_sum = 0, path_max = 0;
     if (wave_tb) {
         uint64_t tiles = 0, longest = 0, work = 0;
@@ -1857,6 +1870,18 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     }
     g2_choose_packed(d, op, sc, eq, et, px.banded);
     if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
+    if (d.wave && !wave_tb && n > 65536 && g2_get_dispatch() == 0) {
+        // as above for the score and start modes (1M pairs GLOBAL 12.7 ms a step, 10.9 of it the device's)
+        uint64_t total = 0, steps = 0;
+        const uint32_t step = n / 4096;
+        for (uint32_t k = 0; k < 4096; k++) {
+            const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
+            total += 64ull * kq * kt;
+            steps += g2_wave_steps(kq, kt);
+        }
+        const double scale = n / 4096.0;
+        if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(0.9 * scale * steps))) d.wave = 0;
+    }
     if (d.wave && !wave_tb) {
         // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
         const bool mixed = op.algo == LOCAL && op.start == WITHOUT_START;

@@ -10,17 +10,19 @@
 // after its last word, and the first lane's row above comes from the records
 // of the pass before: a pair fills its lanes once, whatever its passes.
 //
-// Bound: packed-16 VALU issue, 14 instructions per row pair and step, about 25
-// a step for the hand-over, the ends and the records (1 B written per cell, in
-// whole lines: a record a lane, 64 lanes side by side), times the share of lanes
-// and iterations that hold cells (a pair fills its lanes in GW iterations;
-// strips are rounded up to 2 GW).  Hence 4 lanes wherever the batch has pairs
-// enough, more for few or long ones.  Counters on 300,000 pairs of 100-300 x
-// 100-400 bases: 2.6 G wave instructions, VALU issue 65% of 7.1 ms, 18.7 GB
-// written.  100,000 pairs GLOBAL: 5.95 ms (one lane a pair, direction words) ->
-// 2.3; 50,000 pairs of 50-5000 bases LOCAL 32 -> 9.4 (13.6
-// with the longest on one wave); 50,000 pairs with second
-// best (half a wave a SIMD on two pairs a lane) 5.5 -> 1.6.
+// Bound: the records' writes, 1 B per cell in whole lines (a record a lane, 64
+// lanes side by side), 3 TB/s of them: 100,001 pairs GLOBAL take 2.32 ms, 1.86
+// with a quarter of the records left out and 1.47 with half, and five in a
+// hundred fewer instructions change nothing.  Behind it packed-16 VALU issue, 14
+// instructions per row pair and step and about 25 a step for the hand-over, the
+// ends and the records (2.6 G wave instructions on 300,000 pairs, 65% of 7.1 ms),
+// times the share of lanes and iterations that hold cells: a pair fills its lanes
+// in GW iterations, strips are rounded up to 2 GW.  Hence 4 lanes wherever the
+// batch has pairs enough, more for few or long ones.
+// DP, before and after: 100,001 pairs of 100-300 x 100-400 bases GLOBAL 5.95 ms
+// (one lane a pair, direction words) -> 2.3; 50,000 pairs of 50-5000 bases LOCAL 32
+// -> 9.2 (13.6 with the longest on one wave); 50,000 pairs with second best (half a
+// wave a SIMD on two pairs a lane) 5.5 -> 1.6.
 //
 // The values are those of the lane kernels (k_local_fast, k_global), whose
 // 16-bit bounds the host checks for the batch's largest shape; ends are the
