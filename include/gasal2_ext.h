@@ -91,11 +91,15 @@ uint32_t gasal2_get_cigar(gasal_gpu_storage_t *s, uint32_t k, uint8_t *out, uint
  *   0 auto: long pairs run one wave each, and so does every pair of a
  *     batch of at most 128 pairs per compute unit (64 for WITH_TB), which
  *     the lane path would spread over a fraction of the SIMDs (unless
- *     gasal2_set_wavefront or a tuned entry gives the thresholds);
+ *     gasal2_set_wavefront or a tuned entry gives the thresholds); batches
+ *     that the packed one-wave paths (4 to 256 lanes per pair) run faster
+ *     than the lane kernels take those, WITH_TB while its checkpoints fit in
+ *     the tile budget and in half of the free device memory;
  *   1 reference-order kernels only (one lane per pair, no score tables);
  *   2 one lane per pair only (no one-wave-per-pair path);
  *   3 one wave per pair for every pair the path accepts (LOCAL without
- *     second best, score-only or WITH_TB). */
+ *     second best, score-only or WITH_TB), the packed one-wave paths for
+ *     every batch they accept. */
 void gasal2_set_dispatch(int32_t policy);
 int32_t gasal2_get_dispatch(void);
 
@@ -214,7 +218,7 @@ void gasal2_set_panels(int32_t on);
 /* Which kernel paths the storage's last batch took (no counterpart in the
  * reference; for measurement): bit 0 a packed 16-bit kernel on the
  * one-lane-per-pair path (or KSW's packed row), bit 1 one-wave-per-pair
- * blocks, bit 2 checkpointed traceback on the one-lane-per-pair path. */
+ * blocks, bit 2 checkpointed traceback (lane path or packed one-wave path). */
 int32_t gasal2_last_paths(gasal_gpu_storage_t *storage);
 
 /* Graph mode (default on): each storage captures its device program (pack,
