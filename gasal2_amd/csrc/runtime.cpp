@@ -1626,8 +1626,11 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     g2_choose_fast(d, op, sc, qw, tw);
     // WITH_TB on the packed one-wave path (wavetb.hip); thresholds set by the
     // caller or the tuner keep the kernels they switch.  Its checkpoints may
-    // take half of the device memory free now (this storage's own tile buffer
-    // counted as free: it is reused): about 64 B per tile and 5 KB a pair.
+    // take the tile budget and half of the device memory free now (this
+    // storage's own tile buffer counted as free: it is reused): about 90 B per
+    // tile and 5 KB a pair.  Buffers of 100 GB that grow from batch to batch
+    // cost seconds in the allocator (the full DP of 200,000 pairs of 1-10 kbp in
+    // chunks of 100 to 190 Gcells 8.3 -> 13.4 s with half the memory alone).
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
     if (wave_tb && op.algo == LOCAL && n > 65536 && g2_get_dispatch() == 0) {
@@ -1662,7 +1665,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         wave_tb = least > 0 &&
                   (g2_get_dispatch() == 3 || wave_tb_pays(op, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
                   hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-                  tiles * 90 + (uint64_t)n * 5000 <= ((uint64_t)free_b + m->tb_bytes) / 2;
+                  tiles * 90 + (uint64_t)n * 5000 <= std::min(((uint64_t)free_b + m->tb_bytes) / 2, g_tb_one_size_max);
     }
     uint64_t wf_bytes = 0;   // wave_tb: direction words of the long pairs, within the tile buffer
     // Long LOCAL pairs (score and ends only) run one wave per pair.  The
