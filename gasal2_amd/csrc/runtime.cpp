@@ -1080,20 +1080,21 @@ uint32_t shape8_edge(uint32_t v) {
 // Whether that path beats the lane kernels on a batch.  total and longest:
 // padded cells of the batch and of the longest pair the lane kernels would run;
 // steps: the path's lane-steps on 16 lanes, g2_wave_steps() of every pair.
-// The lane kernels are bound by the longer of the longest pair's serial time
-// and their rate, with part of the shorter one on top; this path by its rate.
-// Constants: 1,000 to 300,000 pairs of 150 x 250 and of 100-300 x 100-400 bases
-// on one MI355X, e.g. LOCAL on the first, this path / lanes: 10,000 pairs
-// 0.33 / 1.07 ms, 100,000 1.56 / 1.74, 300,000 4.0 / 3.6; on the second
-// 100,000 pairs 2.9 / 3.3, 300,000 8.2 / 5.7.
+// The lane kernels take about half of the longest pair's serial time (other
+// launches on the device hide the rest; alone more of it shows) and half of the
+// cells at their rate; this path its lane-steps at its rate.  Lanes / this path
+// among other passes, us: 150 x 250 bases LOCAL 60,000 pairs 965 / 614, 100,000
+// 1114 / 1024, 150,000 1446 / 1548; 100-300 x 100-400 bases GLOBAL 60,000 pairs
+// 1217 / 984, 100,000 1475 / 1653, SEMI_GLOBAL 1445 / 1107 and 1666 / 1859 (alone
+// 2691 / 2584), LOCAL WITH_START 3687 / 2356 and 4480 / 3931.
 bool g2_wave_pays(const G2Opts &op, uint64_t total, uint64_t longest, uint64_t steps) {
     struct Rates { double lane_serial, lane, wave; };   // seconds a cell; cells a second; lane-steps' cells a second
-    const Rates local = {24e-9, 3.2e12, 3.45e12}, local_start = {40e-9, 1.75e12, 2.1e12}, global = {15e-9, 4.1e12, 4.6e12},
+    const Rates local = {24e-9, 3.2e12, 3.45e12}, local_start = {40e-9, 1.75e12, 2.1e12}, global = {15e-9, 4.9e12, 4.6e12},
                 semi = {16e-9, 4.7e12, 4.4e12}, semi_start = {32e-9, 2.4e12, 2.2e12};
     const bool start = op.start == WITH_START;
     const Rates &r = op.algo == LOCAL ? (start ? local_start : local) : (op.algo == GLOBAL ? global : (start ? semi_start : semi));
     const double serial = r.lane_serial * (double)longest, rate = (double)total / r.lane;
-    return (double)steps / r.wave < std::max(serial, rate) + 0.2 * std::min(serial, rate);
+    return 0.8 * (double)steps / r.wave < 0.5 * (serial + rate);
 }
 
 // Cells' worth of lane-steps of a pair on 16 lanes: passes of 256 rows, each
