@@ -1611,11 +1611,12 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     d.eh = m->eh; d.eh_cols = eh_cols;
     d.ksw16 = 0;
     uint64_t ksw_hmax = ~0ull;
-    if (op.algo == KSW && s->host_seed_scores && !px.sub) {   // every KSW value lies in [0, h0 + match * min(Lq, Lt)]
+    if (op.algo == KSW && s->host_seed_scores && !px.sub) {   // every KSW value lies in [0, h0 + best score of a cell * min(Lq, Lt)]
         uint64_t hmax = 0;
+        // a negative mismatch or N penalty adds too
+        const uint64_t up = (uint64_t)std::max({g_scores.match, -g_scores.mismatch, g_scores.has_np ? -g_scores.np : 0, 0});
         for (uint32_t k = 0; k < n; k++)
-            hmax = std::max<uint64_t>(hmax, (uint64_t)s->host_seed_scores[k] +
-                                                (uint64_t)std::max(g_scores.match, 0) * std::min(hq[k], ht[k]));
+            hmax = std::max<uint64_t>(hmax, (uint64_t)s->host_seed_scores[k] + up * std::min(hq[k], ht[k]));
         if (hmax <= 65535 && g_pk16_mode) d.ksw16 = 1;
         ksw_hmax = hmax;
     }
