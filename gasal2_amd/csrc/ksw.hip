@@ -88,7 +88,9 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
     uint32_t redo = 0;                      // the pair needs the row by row kernel
     const int32_t TWm = wave_max<1>(TW);
     int32_t ws = 0, we = wave_max<1>(QW);      // the wave's words
-    for (int32_t s0 = 0; s0 < TWm; s0 += 2) {
+    // we <= ws: no columns left, from the start where every query is empty (their
+    // score is the seed); a sweep stores the column before we
+    for (int32_t s0 = 0; s0 < TWm && ws < we; s0 += 2) {
         const bool act = s0 < TW;
         const int32_t RL = 8 * s0, RH = RL + 8;   // first rows of the two strips
         uint32_t lutL[9], lutH[9];
@@ -256,7 +258,6 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
         const int32_t hi = dead ? 0 : min(QW, last_w + 6);
         ws = max(ws, -wave_max<1>(-lo));
         we = wave_max<1>(hi);
-        if (we <= ws) break;
     }
     if (!ok) return;
     if (redo) {

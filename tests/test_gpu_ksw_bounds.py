@@ -1,6 +1,7 @@
 """KSW where the packed kernels' bounds decide, bit-exact against the oracle: N
 bonuses and mismatch rewards above the match score, on each side of the 4095
-the packed strips hold and of the 65535 the packed row holds."""
+the packed strips hold and of the 65535 the packed row holds; empty queries and
+targets, whole waves of them included."""
 import numpy as np
 import pytest
 
@@ -33,3 +34,14 @@ def test_scores_above_the_match(kind, length):
     scores, n_penalty = ((1, 4, 7, 7), -7) if kind == "n_bonus" else ((1, -7, 7, 7), None)
     b = g.make_batch([q, b"ACGTACGTAC"], [t, b"ACGTACGTTACC"], seeds=np.array([30, 12], np.uint32))
     assert check(b, scores, n_penalty)["score"][0] == 30 + 7 * length
+
+
+@pytest.mark.parametrize("empty", [1, 63, 64, 65, 200])
+def test_empty_sequences(empty):
+    """Sorted last, 64 and more empty queries have a wave to themselves."""
+    rng = np.random.default_rng(9100 + empty)
+    qs = [rng.choice(list(b"ACGT"), int(rng.integers(1, 90))).astype(np.uint8).tobytes() for _ in range(64)]
+    ts = [q[: len(q) // 2] + b"A" + q[len(q) // 2:] for q in qs]
+    qs += [b""] * empty + [b"ACGT", b"ACGTACGTA"]
+    ts += [b"ACGTACGTAC" * int(rng.integers(1, 9)) if k % 3 else b"" for k in range(empty)] + [b"", b"ACGTACGTA"]
+    check(g.make_batch(qs, ts, seeds=rng.integers(0, 40, len(qs)).astype(np.uint32)), (1, 4, 6, 1), 1)
