@@ -91,12 +91,12 @@ struct G2Dev {
     // WITH_TB on that path (wavetb.hip): after wave_coop and wave64 as above, the
     // next wave32 and wave16 slots (whole waves of them, or to the end) on 32 and
     // 16 lanes, the rest on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
-    // and wv_strip (second best) max_tw words a slot, one per strip.
+    // and wv_strip (second best) a word per strip of the batch, places claimed from aux[3].
     uint32_t wave32, wave16;
     uint2 *wv_at;
     uint32_t *wv_strip;
     uint2 *wv_item;                  // second best: strips to recompute (k_second_strips), at most one per strip
-    uint64_t *wv_sec;                // and each slot's answer so far
+    uint64_t *wv_sec;                // and each slot's answer so far (its first place in wv_strip before there is one)
     uint32_t wv_walk;                // a wave walks each pair's path (k_wave_walk), else a lane (k_get_tb)
     // intra-pair wavefront for long pairs (LOCAL score + ends): pairs whose
     // shape passes wf_min_tw / wf_min_cells are sorted first and taken from an

@@ -1788,7 +1788,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         d.wv_at = m->wv_at;
         d.wv_walk = wave_walk_pays((double)path_sum, (double)path_max);
         if (op.second) {
-            ensure(m->wv_strip, m->wv_strip_bytes, (size_t)n * tw * 4);
+            ensure(m->wv_strip, m->wv_strip_bytes, (size_t)wave_strips * 4);
             ensure(m->wv_item, m->wv_item_bytes, (size_t)wave_strips * 8);
             ensure(m->wv_sec, m->wv_sec_bytes, (size_t)n * 8);
             d.wv_strip = m->wv_strip;

@@ -55,6 +55,7 @@ constexpr int WV_WAVES = 4;   // per block
 struct WvShared {
     uint32_t lut16[16];          // score tables of the 16 target nibbles
     uint32_t it0;                // COOP: the pair's first iteration
+    uint32_t strip0;             // and its strips' first record
     int32_t done[WV_WAVES];      // COOP: iterations whose records each wave has stored
     int32_t end[WV_WAVES][4];    // COOP: each wave's best
 };
@@ -84,11 +85,29 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
     uint32_t it0 = 0;
     if (lane == 0 && wv == 0) it0 = atomicAdd(&d.aux[4], COOP ? wv_region((uint32_t)passes, P, WV_WAVES) : (uint32_t)its);
     it0 = __builtin_amdgcn_readfirstlane(it0);
+    // The strips' records of the second best: a place per strip of the batch
+    // (a row of the longest target's strips per pair took n times its length).
+    // k_second_scan finds the pair's first one in wv_sec.
+    uint32_t strip0 = 0;
+    if (SECOND && wv == 0) {
+        const uint32_t own = ok && l == 0 ? (uint32_t)TW : 0u;
+        uint32_t upto = own;
+#pragma unroll
+        for (uint32_t off = 1; off < WAVE; off <<= 1) {
+            const uint32_t o = __shfl_up(upto, off);
+            upto += lane >= (int32_t)off ? o : 0u;
+        }
+        uint32_t first = 0;
+        if (lane == WAVE - 1) first = atomicAdd(&d.aux[3], upto);
+        strip0 = __shfl(__shfl(first, WAVE - 1) + upto - own, lane - l);
+        if (own) d.wv_sec[slot] = strip0;
+    }
     if (COOP) {
-        if (threadIdx.x == 0) sh.it0 = it0;
+        if (threadIdx.x == 0) { sh.it0 = it0; sh.strip0 = strip0; }
         if (lane == 0) sh.done[wv] = 0;
         __syncthreads();
         it0 = __builtin_amdgcn_readfirstlane(sh.it0);
+        if (SECOND) strip0 = __builtin_amdgcn_readfirstlane(sh.strip0);
     }
     uint32_t *out = d.tb + (size_t)(it0 + (COOP ? wv_region((uint32_t)passes, P, (uint32_t)wv) : 0u)) * WV_ITER + (uint32_t)lane * 8u;   // this iteration's records of the lane
     if (ok && l == 0 && wv == 0)
@@ -132,7 +151,7 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
     // a finished strip's maximum (e) joins the pair's
     auto strip_done = [&](int32_t s, uint32_t e, int32_t col, uint32_t low) {
         if (MODE != TB_LOCAL) return;
-        if (SECOND) d.wv_strip[(size_t)slot * d.max_tw + (uint32_t)s] = e | low << 16;
+        if (SECOND) d.wv_strip[(size_t)strip0 + (uint32_t)s] = e | low << 16;
         const int32_t v = (int32_t)(e >> 3);
         if (v > bv) { bv = v; bs = s; bc = col; br = 7 - (int32_t)(e & 7u); }
     };
@@ -351,7 +370,7 @@ __global__ __launch_bounds__(WAVE) void k_second_scan(G2Dev d) {
     if (!census_fast(d.aux[0])) return;
     const uint32_t slot = blockIdx.x * WAVE + threadIdx.x, lane = threadIdx.x;
     const int32_t TW = slot < d.n ? dregs(d.tlen[d.perm[slot]]) : 0;
-    const uint32_t *rec = d.wv_strip + (size_t)(slot < d.n ? slot : 0) * d.max_tw;
+    const uint32_t *rec = d.wv_strip + (slot < d.n ? d.wv_sec[slot] : 0);   // the DP left its place there
     int32_t run = 0, bound = 0;
     for (int32_t s = 0; s < TW; s++) {
         const uint32_t r = rec[s];
