@@ -1627,10 +1627,11 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     const G2Scores &sc = g_scores;
     g2_choose_fast(d, op, sc, qw, tw);
     // WITH_TB on the packed one-wave path (wavetb.hip); thresholds set by the
-    // caller or the tuner keep the kernels they switch.  Its checkpoints may
-    // take the tile budget and half of the device memory free now (this
-    // storage's own tile buffer counted as free: it is reused): about 90 B per
-    // tile and 5 KB a pair.  Buffers of 100 GB that grow from batch to batch
+    // caller or the tuner keep the kernels they switch.  Its checkpoints and
+    // strip records may take the tile budget and half of the device memory free
+    // now (this storage's own buffers counted as free: they are reused).  They
+    // are at least 64 B a tile, which turns large batches away here; below, the
+    // plan's bytes decide.  Buffers of 100 GB that grow from batch to batch
     // cost seconds in the allocator (the full DP of 200,000 pairs of 1-10 kbp in
     // chunks of 100 to 190 Gcells 8.3 -> 13.4 s with half the memory alone).
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
@@ -1648,7 +1649,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         const double scale = n / 4096.0;
         wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, 0.75 * scale * work / 16.0);
     }
-    uint64_t wave_strips = 0, path_sum = 0, path_max = 0;
+    uint64_t wave_strips = 0, path_sum = 0, path_max = 0, wave_room = 0;
     if (wave_tb) {
         uint64_t tiles = 0, longest = 0, work = 0;
         uint32_t least = 0xFFFFFFFFu;
@@ -1666,15 +1667,17 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         size_t free_b = 0, total_b = 0;
         wave_tb = least > 0 &&
                   (g2_get_dispatch() == 3 || wave_tb_pays(op, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
-                  hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-                  tiles * 90 + (uint64_t)n * 5000 <= std::min(((uint64_t)free_b + m->tb_bytes) / 2, g_tb_one_size_max);
+                  hipMemGetInfo(&free_b, &total_b) == hipSuccess;
+        wave_room = std::min(((uint64_t)free_b + m->tb_bytes + m->wv_strip_bytes + m->wv_item_bytes) / 2, g_tb_one_size_max);
+        wave_tb = wave_tb && tiles * 64 <= wave_room;
     }
     uint64_t wf_bytes = 0;   // wave_tb: direction words of the long pairs, within the tile buffer
     // Long LOCAL pairs (score and ends only) run one wave per pair.  The
     // device applies the same shape test in k_keys and also needs the nibble
     // census to allow the score tables; the host count only sizes the launch.
     uint32_t eq = qw, et = tw;   // largest shape the one-lane-per-pair kernels see
-    uint32_t nlong = 0;
+    uint32_t nlong = 0, ltw = 0, lqw = 0;
+    uint64_t wtot = 0;   // 32-byte tiles of the long pairs
     bool switched = g_wf_user;   // lane / one-wave thresholds set by the caller or the tuner
     if (d.fast && op.algo == LOCAL && (op.start == WITHOUT_START || (op.start == WITH_TB && !px.banded)) && !op.second &&
         g2_get_dispatch() != 2) {
@@ -1702,9 +1705,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         const bool all = g2_get_dispatch() == 3 || few;
         d.wf_min_tw = all ? 1u : min_tw;
         d.wf_min_cells = all ? 0u : min_cells;
-        uint32_t ltw = 0, lqw = 0, sq = 0, st = 0;
-        const bool wtb = op.start == WITH_TB;
-        uint64_t wtot = 0;   // 32-byte tiles of the long pairs
+        uint32_t sq = 0, st = 0;
         // no pair can pass the shape test when the largest shapes do not
         const bool any_long = tw >= d.wf_min_tw && (uint64_t)qw * tw * 64u >= (uint64_t)d.wf_min_cells;
         for (uint32_t k = 0; any_long && k < n; k++) {
@@ -1713,7 +1714,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
                 nlong++;
                 ltw = std::max(ltw, kt);
                 lqw = std::max(lqw, kq);
-                if (wtb) wtot += (uint64_t)kq * kt;
+                wtot += (uint64_t)kq * kt;
             } else {
                 sq = std::max(sq, kq);
                 st = std::max(st, kt);
@@ -1723,36 +1724,50 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             eq = std::max(sq, 1u);
             et = std::max(st, 1u);
             d.wf_blocks = std::min<uint32_t>(nlong, max_blocks);
-            d.wf_stride = ((ltw + 63) / 64) * 17 * 64;
-            if (8 * qw > 1024) {   // more than one column block: strip state is saved between blocks
-                ensure(m->wf, m->wf_bytes, (size_t)d.wf_blocks * d.wf_stride * 4);
-                d.wf_scratch = m->wf;
-            } else {
-                d.wf_stride = 0;
-                d.wf_scratch = nullptr;
-            }
-            if (wave_tb) {   // run only when the census refuses the score tables
-                wf_bytes = wtot * 32;
-                ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
-                d.wf_tbo = m->wf_tbo;
-            } else if (wtb) {   // per-pair direction tiles (or checkpoints) of the long pairs; the waves claim their places
-                // checkpoints take twice the bytes of direction words: only while
-                // they fit in 80% of the device memory free now (this storage's
-                // own buffer counted as free: it is reused)
-                size_t free_b = 0, total_b = 0;
-                const bool room = g_tb_ckpt == 2 && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-                                  wtot * 64 <= ((uint64_t)free_b + m->wf_tb_bytes) / 10 * 8;
-                const bool wck = g_tb_ckpt == 2 && room &&
-                                 (uint64_t)std::max(g_scores.match, 0) * 8u * std::min(lqw, ltw) <= 32767u &&
-                                 (uint64_t)g_scores.gapoe +
-                                         (uint64_t)std::max(std::max(g_scores.mismatch, g_scores.has_np ? g_scores.np : 0), 0) <=
-                                     32767u;
-                ensure(m->wf_tb, m->wf_tb_bytes, (size_t)wtot * 32 * (wck ? 2 : 1) + 256);
-                ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
-                d.wf_tb = m->wf_tb;
-                d.wf_tbo = m->wf_tbo;
-                if (wck) d.wf_tbh = m->wf_tb + wtot * 8;
-            }
+        }
+    }
+    uint64_t wave_bytes = 0;
+    if (wave_tb) {
+        wave_bytes = wave_tb_plan(m, d, hq, ht, n, qw, tw) * 8192;
+        // with the allocator's slack (ensure)
+        const uint64_t need = wave_bytes + (op.second ? wave_strips * 12 : 0);
+        if (need + need / 8 > wave_room || wave_strips > 0xFFFFFFFFull) {
+            wave_tb = false;
+            wave_bytes = 0;
+            d.wave_coop = d.wave64 = d.wave32 = d.wave16 = 0;
+        }
+    }
+    if (nlong) {
+        const bool wtb = op.start == WITH_TB;
+        d.wf_stride = ((ltw + 63) / 64) * 17 * 64;
+        if (8 * qw > 1024) {   // more than one column block: strip state is saved between blocks
+            ensure(m->wf, m->wf_bytes, (size_t)d.wf_blocks * d.wf_stride * 4);
+            d.wf_scratch = m->wf;
+        } else {
+            d.wf_stride = 0;
+            d.wf_scratch = nullptr;
+        }
+        if (wave_tb) {   // run only when the census refuses the score tables
+            wf_bytes = wtot * 32;
+            ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
+            d.wf_tbo = m->wf_tbo;
+        } else if (wtb) {   // per-pair direction tiles (or checkpoints) of the long pairs; the waves claim their places
+            // checkpoints take twice the bytes of direction words: only while
+            // they fit in 80% of the device memory free now (this storage's
+            // own buffer counted as free: it is reused)
+            size_t free_b = 0, total_b = 0;
+            const bool room = g_tb_ckpt == 2 && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+                              wtot * 64 <= ((uint64_t)free_b + m->wf_tb_bytes) / 10 * 8;
+            const bool wck = g_tb_ckpt == 2 && room &&
+                             (uint64_t)std::max(g_scores.match, 0) * 8u * std::min(lqw, ltw) <= 32767u &&
+                             (uint64_t)g_scores.gapoe +
+                                     (uint64_t)std::max(std::max(g_scores.mismatch, g_scores.has_np ? g_scores.np : 0), 0) <=
+                                 32767u;
+            ensure(m->wf_tb, m->wf_tb_bytes, (size_t)wtot * 32 * (wck ? 2 : 1) + 256);
+            ensure(m->wf_tbo, m->wf_tbo_bytes, (size_t)n * 8);
+            d.wf_tb = m->wf_tb;
+            d.wf_tbo = m->wf_tbo;
+            if (wck) d.wf_tbh = m->wf_tb + wtot * 8;
         }
     }
     // BANDED in packed halves: E and F are held at or above 0, so every value
@@ -1781,9 +1796,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     }
     // The packed one-wave path's checkpoints and the direction words of the
     // kernels that run when the census refuses the score tables share one buffer.
-    uint64_t wave_bytes = 0;
     if (wave_tb) {
-        wave_bytes = wave_tb_plan(m, d, hq, ht, n, qw, tw) * 8192;
         ensure(m->wv_at, m->wv_at_bytes, (size_t)n * 8);
         d.wv_at = m->wv_at;
         d.wv_walk = wave_walk_pays((double)path_sum, (double)path_max);

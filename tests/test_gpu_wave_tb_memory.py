@@ -50,3 +50,22 @@ def test_strip_records_of_one_long_target():
     assert took < (2500 * 12 + 98 * 260) * 8192 * 9 / 8 + 3e8, took
     lane, _, _ = run(b, g.LOCAL, True, 2)
     assert_same(got, lane, fields(g.LOCAL, g.WITH_TB, True) + ["n_ops", "cigars"], "lane path")
+
+
+@pytest.mark.parametrize("algo,second", [(g.LOCAL, False), (g.LOCAL, True), (g.GLOBAL, False)])
+def test_tile_budget_holds_for_short_queries(algo, second):
+    """A pass lasts at least as many iterations as the group has lanes: 200
+    queries of 20 bases against 14,000 want 400 MB of checkpoints and more for
+    34 MB of tiles.  Over the budget the lane kernels run."""
+    rng = np.random.default_rng(8200)
+    t = rng.choice(list(b"ACGT"), 14_000).astype(np.uint8)
+    b = g.make_batch([t[o:o + 20].tobytes() for o in rng.integers(0, 13_000, 200)], [t.tobytes()] * 200)
+    budget = 100_000_000
+    g.lib().gasal2_set_tile_budget(budget)
+    try:
+        got, took, _ = run(b, algo, second, 3)
+    finally:
+        g.lib().gasal2_set_tile_budget(64 << 30)
+    assert took < budget * 9 / 8 + 1.5e8, took
+    lane, _, _ = run(b, algo, second, 2)
+    assert_same(got, lane, fields(algo, g.WITH_TB, second) + ["n_ops", "cigars"], "lane path")
