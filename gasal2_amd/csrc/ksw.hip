@@ -67,15 +67,10 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
     const int32_t qlen = ok ? (int32_t)d.qlen[pr] : 0, tlen = ok ? (int32_t)d.tlen[pr] : 0;
     const int32_t QW = dregs((uint32_t)qlen), TW = dregs((uint32_t)tlen);
     const uint32_t *Qp = d.pq + (d.qoff[pr] >> 3), *Tp = d.pt + (d.toff[pr] >> 3);
-    uint32_t ps = 1;
-    int32_t q_last = max(QW - 1, 0), t_last = max(TW - 1, 0);   // words the pair holds
-    if (d.qpan) {
-        Qp = d.qpan + (size_t)grp * d.qpan_w * WAVE + lane;
-        Tp = d.tpan + (size_t)grp * d.tpan_w * WAVE + lane;
-        ps = WAVE;
-        q_last = (int32_t)d.qpan_w - 1;
-        t_last = (int32_t)d.tpan_w - 1;
-    }
+    // a word in eight columns of sixteen rows: transposed panels gain nothing
+    // (200,000 pairs 2.37 ms with them, 2.34 without) and take a row of the
+    // longest target's words for every pair
+    const int32_t q_last = max(QW - 1, 0), t_last = max(TW - 1, 0);   // words the pair holds
     uint32_t *__restrict__ bd = d.bnd + (size_t)grp * d.bnd_cols * WAVE + lane;
     const int32_t h0 = ok ? (int32_t)d.seeds[pr] : 0;
     const int32_t gapo = c.gapo, gape = c.gape, gapoe = c.gapoe;
@@ -95,7 +90,7 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
         const int32_t RL = 8 * s0, RH = RL + 8;   // first rows of the two strips
         uint32_t lutL[9], lutH[9];
         {
-            const uint32_t gL = Tp[(size_t)min(s0, t_last) * ps], gH = Tp[(size_t)min(s0 + 1, t_last) * ps];
+            const uint32_t gL = Tp[min(s0, t_last)], gH = Tp[min(s0 + 1, t_last)];
 #pragma unroll
             for (int m = 1; m < 9; m++) {   // rows past the target score -8: they raise no maximum
                 lutL[m] = RL + m - 1 < tlen ? lut16[(gL >> (32 - 4 * m)) & 15u] : 0x88888888u;
@@ -179,7 +174,7 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
                 return bottom;
             };
             uint32_t nxt[8];
-            uint32_t qn = Qp[(size_t)min(ws, q_last) * ps];
+            uint32_t qn = Qp[min(ws, q_last)];
             auto fetch = [&](int32_t j) {
                 const uint32_t *p = bd + (size_t)(8 * j) * WAVE;
 #pragma unroll
@@ -192,7 +187,7 @@ __global__ __launch_bounds__(64) void k_ksw_pk(G2Dev d, G2Scores c, int32_t end_
                 for (int kk = 0; kk < 8; kk++) cur[kk] = nxt[kk];
                 const uint32_t q = qn;
                 fetch(min(j + 1, we - 1));
-                qn = Qp[(size_t)min(j + 1, q_last) * ps];
+                qn = Qp[min(j + 1, q_last)];
                 if (s0 == 0) {   // above row 0 (:78-81)
 #pragma unroll
                     for (int kk = 0; kk < 8; kk++) cur[kk] = (uint32_t)max(h0 - gapoe - gape * (8 * j + kk), 0);

@@ -1783,9 +1783,9 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         sc.gape >= 0 && sc.gape <= 255 && sc.gapoe >= 1 && sc.gapoe <= 16000 && op.ksw_eb <= sc.gapoe &&
         8ull * qw + 8 <= 65535)
         d.ksw_pk = 1;
-    // Transposed sequence panels for the fast LOCAL and KSW lane path (k_panel):
+    // Transposed sequence panels for the fast LOCAL lane path (k_panel):
     // groups after the long pairs, eq query words and et target words each.
-    if (g_panels && (d.ksw_pk || (d.fast && op.algo == LOCAL)) && !px.banded && !wave_tb && n > nlong) {
+    if (g_panels && d.fast && op.algo == LOCAL && !px.banded && !wave_tb && n > nlong) {
         const uint64_t lgroups = ((uint64_t)(n - nlong) + 63) / 64;
         ensure(m->qpan, m->qpan_bytes, (size_t)(lgroups * eq * 256) + 256);
         ensure(m->tpan, m->tpan_bytes, (size_t)(lgroups * et * 256) + 256);

@@ -1,9 +1,10 @@
 """KSW where the packed kernels' bounds decide, bit-exact against the oracle: N
 bonuses and mismatch rewards above the match score, on each side of the 4095
 the packed strips hold and of the 65535 the packed row holds; empty queries and
-targets, whole waves of them included."""
+targets, whole waves of them included; one long target among short ones."""
 import numpy as np
 import pytest
+import torch
 
 import gasal2_amd as g
 import pyoracle as O
@@ -45,3 +46,28 @@ def test_empty_sequences(empty):
     qs += [b""] * empty + [b"ACGT", b"ACGTACGTA"]
     ts += [b"ACGTACGTAC" * int(rng.integers(1, 9)) if k % 3 else b"" for k in range(empty)] + [b"", b"ACGTACGTA"]
     check(g.make_batch(qs, ts, seeds=rng.integers(0, 40, len(qs)).astype(np.uint32)), (1, 4, 6, 1), 1)
+
+
+def test_memory_of_one_long_target():
+    """40,000 short pairs and a target of 100,000 bases: nothing is sized by the
+    number of pairs times the longest target (2 GB of words)."""
+    rng = np.random.default_rng(9300)
+    t = rng.choice(list(b"ACGT"), 100_000).astype(np.uint8)
+    qs = [t[o:o + 40].tobytes() for o in rng.integers(0, 1000, 40_000)]
+    ts = [q[:25] + b"AC" + q[25:] for q in qs]
+    ts[777] = t.tobytes()
+    b = g.make_batch(qs, ts, seeds=rng.integers(0, 30, 40_000).astype(np.uint32))
+    a = g.Aligner(g.Parameters(algo=g.KSW), 40, 100_000, b.n)
+    try:
+        a.load(b, per_pair=False)
+        free = torch.cuda.mem_get_info()[0]
+        a.run_resident()
+        a.sync()
+        took = free - torch.cuda.mem_get_info()[0]
+        got = a.download()
+    finally:
+        a.close()
+    assert took < 3e8, took
+    ref = O.align(b, g.KSW)
+    for f in FIELDS:
+        assert np.array_equal(got[f], ref[f]), f
