@@ -1077,7 +1077,7 @@ __device__ void lane_local_pk(const G2Dev &d, const G2Scores &c, const LaneCtx &
     if (with_start) local_reverse_start(d, c, x, census, bv, bv > 0 ? bc : 0, bv > 0 ? bs * 8 + br : 0);
 }
 
-template <bool LOCALT>
+template <bool LOCALT, bool WV>
 __device__ void tb_walk(const G2Dev &d, const G2Scores &c, uint32_t slot, const uint32_t *lut16, bool fused);
 
 // CK (WITH_TB only): checkpointed traceback.  No direction words: per 8x8
@@ -1266,7 +1266,7 @@ __global__ __launch_bounds__(64) void k_local_fast(G2Dev d, G2Scores c) {
     if (START == S_WITH_START) local_reverse_start(d, c, x, census, vbest, maxXY_x, maxXY_y);
     if (CK && d.tb_fused) {
         __threadfence();   // this lane's checkpoints and results, seen by its own loads
-        tb_walk<true>(d, c, x.slot, lut16, true);
+        tb_walk<true, false>(d, c, x.slot, lut16, true);
     }
 }
 
@@ -2540,7 +2540,10 @@ __device__ __forceinline__ uint32_t seq_word4(const uint32_t *arr, uint32_t a, u
 // One pair's walk (the body of k_get_tb), for the pair in sorted slot `slot`.
 // fused: called by k_local_fast<.., CK> right after the pair's DP, which walks
 // exactly the pairs whose tiles it checkpointed; k_get_tb then skips those.
-template <bool LOCALT>
+// WV: every pair ran on the packed one-wave path (wavetb.hip).  One body for both
+// held three formats at once: 96 VGPRs and 84 B of scratch for GLOBAL, 52 and none
+// without that path's, and 56 B against 20 for LOCAL.
+template <bool LOCALT, bool WV>
 __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint32_t slot, const uint32_t *lut16,
                                         bool fused) {
     if (slot >= d.n) return;
@@ -2548,10 +2551,8 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     // long pairs (sorted first) ran one wave per pair with per-pair tiles; the
     // lane path's groups count from the first slot after them
     const uint32_t census = d.aux[0];
-    // every pair ran on the packed one-wave path (wavetb.hip)
-    const bool wv = d.wave && census_fast(census);
-    if (wv && d.wv_walk) return;   // walked by k_wave_walk
-    const uint32_t nlong = (LOCALT && d.wf_tb && !wv) ? d.aux[2] : 0u;
+    if (WV != (d.wave && census_fast(census))) return;
+    const uint32_t nlong = (LOCALT && !WV && d.wf_tb) ? d.aux[2] : 0u;
     const bool wfp = slot < nlong;
     const uint32_t rslot = slot - nlong;
     const uint32_t lane = rslot & (WAVE - 1), grp = rslot / WAVE;
@@ -2560,7 +2561,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     // LOCAL words written by k_local_fast carry the four comparisons as
     // "not" bits; the match/mismatch label comes from the bases.
     // banded runs (k_local_band) store band-compressed tiles per pair
-    const bool band = LOCALT && d.band_lo != nullptr;
+    const bool band = LOCALT && !WV && d.band_lo != nullptr;
     const int32_t blo = band ? d.band_lo[pr] : 0, bhi = band ? d.band_hi[pr] : 0;
     const int32_t bbw = band ? (int32_t)d.band_bw[pr] : 0;
     uint32_t bflag = 0;
@@ -2569,13 +2570,13 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     const bool lanefast = d.fast && d.enc_ok && census_fast(census);
     const bool fastfmt = !LOCALT || band || wfp || lanefast;
     // lane-path tiles of k_local_fast<.., CK> are recomputed from checkpoints
-    const bool ck = LOCALT && !band && !wfp && !wv && lanefast && d.tbh != nullptr;
+    const bool ck = LOCALT && !band && !wfp && !WV && lanefast && d.tbh != nullptr;
     // long pairs of k_local_fast's one-wave blocks with checkpoints (wf_local<.., CK>)
     const bool wck = LOCALT && wfp && d.wf_tbh != nullptr && census_fast(census);
     if (fused ? !ck : (ck && d.tb_fused)) return;   // walked by k_local_fast, or not fused there
     // recomputed tiles hold the reference's nibbles; stored sign-bit words are decoded
-    const bool decode = fastfmt && !ck && !wck && !wv;
-    const uint2 wv_at = wv ? d.wv_at[pr] : make_uint2(0u, 0u);
+    const bool decode = fastfmt && !ck && !wck && !WV;
+    const uint2 wv_at = WV ? d.wv_at[pr] : make_uint2(0u, 0u);
     const uint32_t qw0 = d.qoff[pr] >> 3;
     const uint32_t *Qw = d.pq + qw0, *Tw = d.pt + (d.toff[pr] >> 3);
     uint4 q4 = {0u, 0u, 0u, 0u};   // recompute walks: cached query words
@@ -2621,7 +2622,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
             } else if (wfp && !wck) {
                 chunk = d.wf_tb + (d.wf_tbo[pr] + (size_t)strip * QW + (size_t)word) * 8;
             }
-            if (ck || wck || wv) {
+            if (ck || wck || WV) {
                 if (strip != lut_key) {   // the walk stays in one strip for several tiles
                     lut_key = strip;
                     const uint32_t gw = Tw[strip];
@@ -2633,7 +2634,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
                     const TbView lv = tb_view(d, grp, lane), hv = tb_view(d, grp, lane, d.tbh);
                     if (strip > 0) hv.load(strip - 1, word, top);
                     lv.load(strip, word, left);
-                } else if (wv) {
+                } else if (WV) {
                     if (strip > 0) tb_load(wv_tile(d, wv_at, QW, strip - 1, word, WV_BOTTOM), top);
                     tb_load(wv_tile(d, wv_at, QW, strip, word, WV_LEFT), left);
                 } else {   // per pair [strip][word] x 8, H and E of the same column
@@ -2661,7 +2662,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
             }
             ch_key = key;
         }
-        if (LOCALT && (ck || wck || wv)) {
+        if (LOCALT && (ck || wck || WV)) {
             // recomputed tiles: reference nibbles, and a LOCAL walk stays inside
             // the matrix, so a step reads the column's word (re-selected only on
             // a column move) and the tile changes when i >> 3 or j >> 3 does
@@ -2752,18 +2753,18 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     if (band && bflag) d.band_flags[pr] |= (uint8_t)bflag;
 }
 
-template <bool LOCALT>
+template <bool LOCALT, bool WV>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_get_tb(G2Dev d, G2Scores c) {
     // score table of each target nibble for the tile recompute (one per block,
     // built before any thread leaves)
     __shared__ uint32_t lut16[16];
-    if (LOCALT || d.wave) {
+    if (LOCALT || WV) {
         if (threadIdx.x < 16)
             lut16[threadIdx.x] = LOCALT ? score_lut(c, c.has_np ? -c.np : 0, d.aux[0], threadIdx.x)
                                         : score_lut<true>(c, 0, d.aux[0], threadIdx.x);
         __syncthreads();
     }
-    tb_walk<LOCALT>(d, c, blockIdx.x * blockDim.x + threadIdx.x, lut16, false);
+    tb_walk<LOCALT, WV>(d, c, blockIdx.x * blockDim.x + threadIdx.x, lut16, false);
 }
 
 // Copies each pair's CIGAR to the reference's layout (bytes at the pair's query
@@ -3053,9 +3054,12 @@ hipError_t g2_run(const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStrea
         if (d.wave && d.wv_walk) {
             const hipError_t e = g2_wave_walk(sc, op, d, s);
             if (e != hipSuccess) return e;
+        } else if (d.wave) {
+            if (op.algo == A_LOCAL) k_get_tb<true, true><<<grid, blk, 0, s>>>(d, sc);
+            else k_get_tb<false, true><<<grid, blk, 0, s>>>(d, sc);
         }
-        if (op.algo == A_LOCAL) k_get_tb<true><<<grid, blk, 0, s>>>(d, sc);
-        else if (op.algo == A_GLOBAL) k_get_tb<false><<<grid, blk, 0, s>>>(d, sc);
+        if (op.algo == A_LOCAL) k_get_tb<true, false><<<grid, blk, 0, s>>>(d, sc);
+        else if (op.algo == A_GLOBAL) k_get_tb<false, false><<<grid, blk, 0, s>>>(d, sc);
         else k_no_tb<<<nb256, 256, 0, s>>>(d);
         G2_LAUNCH_CHECK();
         if (d.cigar_qlayout) {
