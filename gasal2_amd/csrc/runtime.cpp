@@ -1637,8 +1637,10 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
     if (wave_tb && op.algo == LOCAL && n > 65536 && g2_get_dispatch() == 0) {
-        // a large batch that the lane kernels clearly run faster is told by 4096
-        // of its pairs (a pass over 1M pairs took 2 ms of a 24.7 ms step)
+        // a large batch that the lane kernels run faster is told by 4096 of its
+        // pairs, with the longest shapes as one pair's (a pass over 1M pairs took
+        // 2 ms of a 24.7 ms step; 300,000 pairs with second best 0.72 ms of host
+        // time a pass where the sample left all but clear cases to the sums, 0.15 so)
         uint64_t tiles = 0, work = 0;
         const uint32_t step = n / 4096;
         for (uint32_t k = 0; k < 4096; k++) {
@@ -1647,7 +1649,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             work += wave_tb_iters(kq, kt, 4);
         }
         const double scale = n / 4096.0;
-        wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, 0.75 * scale * work / 16.0);
+        wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
     }
     uint64_t wave_strips = 0, path_sum = 0, path_max = 0, wave_room = 0;
     if (wave_tb) {
@@ -1898,7 +1900,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             steps += g2_wave_steps(kq, kt);
         }
         const double scale = n / 4096.0;
-        if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(0.9 * scale * steps))) d.wave = 0;
+        if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(scale * steps))) d.wave = 0;
     }
     if (d.wave && !wave_tb) {
         // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
