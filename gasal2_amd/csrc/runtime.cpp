@@ -1056,12 +1056,19 @@ bool wave_tb_pays(const G2Opts &op, double cells, double longest, double work) {
     return work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
 }
 
-// Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb): the
-// longest path's serial time (1.6 us a cell on a lane, 0.1 on a wave) against
-// the sum's (11 ps a cell on lanes, 62 on waves).  Lanes / waves: 64 pairs of
-// 100-300 bases 486 / 53 us, 51,000 617 / 638, 120,000 727 / 1432; 50,000 pairs
-// of 50-5000 bases 8.7 / 1.6 ms.
-bool wave_walk_pays(double sum, double longest) { return 40e-6 + 51e-12 * sum < 1.6e-6 * longest; }
+// Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb), of n
+// paths: their cells on the diagonal and in gaps (GLOBAL's lengths differ by at
+// least those), the longest path's and the most gaps.  A lane takes 0.7 us a cell
+// whatever it is, and hides most of the others' walks behind the longest.  A wave
+// steps over a stretch of matches at once, 38 ps a cell of the sum, and over
+// gaps one by one, 150 ps of the sum and 0.4 us of the longest.  Lanes / waves, us:
+// 100 x 100 bases 10,000 pairs 88 / 56, 60,000 126 / 272; 250 x 250 10,000 201 /
+// 147, 60,000 235 / 621; 1500 x 1500 1000 pairs 1161 / 139; GLOBAL 2000 x 60 1000
+// pairs 1246 / 784, 10,000 1323 / 3387; 30 x 300 1000 231 / 142, 10,000 242 / 374.
+bool wave_walk_pays(double n, double diag, double gaps, double longest, double most_gaps) {
+    const double waves = 15e-6 + std::max(1e-9 * n + 38e-12 * diag + 150e-12 * gaps, 0.4e-6 * most_gaps);
+    return waves < 10e-6 + 0.7e-6 * longest + 11e-12 * (diag + gaps);
+}
 
 // Shape buckets as the device sorts by them (k_keys), and a bucket's largest x.
 uint32_t shape8(uint32_t x) {
@@ -1651,7 +1658,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         const double scale = n / 4096.0;
         wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
     }
-    uint64_t wave_strips = 0, path_sum = 0, path_max = 0, wave_room = 0;
+    uint64_t wave_strips = 0, path_diag = 0, path_gaps = 0, wave_room = 0;
+    uint32_t path_max = 0, gaps_max = 0;
     if (wave_tb) {
         uint64_t tiles = 0, longest = 0, work = 0;
         uint32_t least = 0xFFFFFFFFu;
@@ -1662,9 +1670,11 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             longest = std::max(longest, (uint64_t)kq * kt);
             work += wave_tb_iters(kq, kt, 4);
             wave_strips += kt;
-            const uint32_t path = op.algo == LOCAL ? std::min(hq[k], ht[k]) : std::max(hq[k], ht[k]);
-            path_sum += path;
-            path_max = std::max<uint64_t>(path_max, path);
+            const uint32_t diag = std::min(hq[k], ht[k]), gaps = op.algo == LOCAL ? 0 : std::max(hq[k], ht[k]) - diag;
+            path_diag += diag;
+            path_gaps += gaps;
+            path_max = std::max(path_max, diag + gaps);
+            gaps_max = std::max(gaps_max, gaps);
         }
         size_t free_b = 0, total_b = 0;
         wave_tb = least > 0 &&
@@ -1801,7 +1811,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     if (wave_tb) {
         ensure(m->wv_at, m->wv_at_bytes, (size_t)n * 8);
         d.wv_at = m->wv_at;
-        d.wv_walk = wave_walk_pays((double)path_sum, (double)path_max);
+        d.wv_walk = wave_walk_pays(n, (double)path_diag, (double)path_gaps, path_max, gaps_max);
         if (op.second) {
             ensure(m->wv_strip, m->wv_strip_bytes, (size_t)wave_strips * 4);
             ensure(m->wv_item, m->wv_item_bytes, (size_t)wave_strips * 8);
