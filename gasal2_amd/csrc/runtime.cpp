@@ -1042,17 +1042,21 @@ uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double load, double longest4) {
     return best;
 }
 
-// Whether LOCAL WITH_TB runs there: padded cells, the longest pair's, and the
-// path's wave-iterations on 4 lanes.  The lane kernels (two pairs a lane) are
+// Whether WITH_TB runs there: pairs, padded cells, the longest pair's, and the
+// path's wave-iterations on 4 lanes.  LOCAL: the lane kernels (two pairs a lane) are
 // bound by the longest pair's serial time, part of which other launches on the
 // device can hide, and their rate; that path by its rate, the second best's
 // strips included.  100-300 x 100-400 bases with second best, lanes / that path:
 // 30,000 pairs 6.2 / 1.8 ms, 100,000 6.4 / 3.5, 300,000 11.0 / 9.3 alone and 7.9 /
 // 8.2 among other passes, 900,000 19.5 / 26.8; 150 x 250 without: 100,000 pairs
-// 3.0 / 2.0, 300,000 5.7 / 5.0, 1,000,000 15.7 / 17.0.  GLOBAL always does: its
-// lanes store direction words in 32 bits, 900,000 pairs 26.4 / 23.9 ms.
-bool wave_tb_pays(const G2Opts &op, double cells, double longest, double work) {
-    if (op.algo == GLOBAL) return true;
+// 3.0 / 2.0, 300,000 5.7 / 5.0, 1,000,000 15.7 / 17.0.  GLOBAL: its lanes store
+// direction words in 32 bits, whatever the pair's shape, where a wave's pass has
+// five iterations at least and the host plans every pair.  Lanes / that path, a
+// pass with its host time: 100-300 x 100-400 bases 900,000 pairs 26.4 / 23.9 ms;
+// 100 x 100 60,000 0.94 / 0.75, 150,000 1.42 / 1.58; 48 x 48 10,000 235 / 228 us,
+// 60,000 331 / 514; 16 x 16 1000 109 / 144, 600,000 427 / 2947.
+bool wave_tb_pays(const G2Opts &op, double n, double cells, double longest, double work) {
+    if (op.algo == GLOBAL) return 30e-6 + 4e-9 * n + work * 8192.0 / 2.95e12 < 36e-9 * longest + cells / 1.9e12;
     return work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
 }
 
@@ -1643,7 +1647,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // chunks of 100 to 190 Gcells 8.3 -> 13.4 s with half the memory alone).
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
-    if (wave_tb && op.algo == LOCAL && n > 65536 && g2_get_dispatch() == 0) {
+    if (wave_tb && n > 65536 && g2_get_dispatch() == 0) {
         // a large batch that the lane kernels run faster is told by 4096 of its
         // pairs, with the longest shapes as one pair's (a pass over 1M pairs took
         // 2 ms of a 24.7 ms step; 300,000 pairs with second best 0.72 ms of host
@@ -1656,7 +1660,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             work += wave_tb_iters(kq, kt, 4);
         }
         const double scale = n / 4096.0;
-        wave_tb = wave_tb_pays(op, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
+        wave_tb = wave_tb_pays(op, n, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
     }
     uint64_t wave_strips = 0, path_diag = 0, path_gaps = 0, wave_room = 0;
     uint32_t path_max = 0, gaps_max = 0;
@@ -1678,7 +1682,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         }
         size_t free_b = 0, total_b = 0;
         wave_tb = least > 0 &&
-                  (g2_get_dispatch() == 3 || wave_tb_pays(op, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
+                  (g2_get_dispatch() == 3 || wave_tb_pays(op, n, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
                   hipMemGetInfo(&free_b, &total_b) == hipSuccess;
         wave_room = std::min(((uint64_t)free_b + m->tb_bytes + m->wv_strip_bytes + m->wv_item_bytes) / 2, g_tb_one_size_max);
         wave_tb = wave_tb && tiles * 64 <= wave_room;
