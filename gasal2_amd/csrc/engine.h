@@ -161,7 +161,9 @@ void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t e
 uint32_t g2_wave_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_t tw, int32_t fast);
 bool g2_wave_pays(const G2Opts &op, uint64_t total, uint64_t longest, uint64_t steps);
 uint64_t g2_wave_steps(uint32_t qw, uint32_t tw);
-int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total);
+uint32_t g2_cu_count();           // compute units of the current device
+constexpr double G2_WAVE_COOP = 2.3e-4;   // least share of a pair on a block of four waves
+int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total, double coop);
 G2Scores g2_scores();
 
 // Dispatch policy for LOCAL (0 auto, 1 reference-order kernel only).

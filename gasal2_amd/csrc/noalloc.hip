@@ -192,7 +192,7 @@ extern "C" int32_t gasal2_aln_noalloc(const void *query_batch, const void *targe
     d.wave = g2_wave_fits(op, sc, qw, tw, d.fast);
     if (d.wave && (g2_get_dispatch() == 3 ||
                    (g2_get_dispatch() == 0 && g2_wave_pays(op, total, cells, g2_wave_steps(qw, tw) * n)))) {
-        const int lanes = g2_wave_lanes(qw, tw, total);
+        const int lanes = g2_wave_lanes(qw, tw, total, n <= 4 * g2_cu_count() ? G2_WAVE_COOP : 2.0);
         d.wave_coop = lanes == 256 ? n : 0;
         d.wave64 = lanes == 64 ? n : 0;
     } else {

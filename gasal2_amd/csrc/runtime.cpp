@@ -52,7 +52,9 @@ constexpr uint32_t WF_TB_MIN_TW = 32, WF_TB_MIN_CELLS = 1u << 18;
 // Measured on 150 x 250-base pairs: the one-wave path wins below about 160
 // pairs per CU for score-only LOCAL and below about 86 for WITH_TB.
 constexpr uint32_t WF_FEW_PER_CU = 128, WF_FEW_PER_CU_TB = 64;
-// compute units of the current device (cached per device)
+}  // namespace
+
+// cached per device
 uint32_t g2_cu_count() {
     static std::atomic<uint32_t> cache[64];
     int dev = 0;
@@ -66,6 +68,8 @@ uint32_t g2_cu_count() {
     }
     return v;
 }
+
+namespace {
 int g_graph_mode = 1;   // capture the device program per batch shape and replay it
 uint64_t g_tb_one_size_max = 64ull << 30;   // lane-path tiles: one size for all groups up to this many bytes
 int g_tb_ckpt = 1;   // checkpointed traceback: 1 the fast LOCAL WITH_TB lane path, 2 also one-wave pairs
@@ -1116,8 +1120,10 @@ uint64_t g2_wave_steps(uint32_t qw, uint32_t tw) { return 2048ull * ((tw + 31) /
 // would otherwise outlast its share of a batch of `total` cells, 64 also where
 // the share of lanes and steps that hold cells is close to that of 16 lanes.
 // Measured on 20,000 pairs of 50-5000 bases, LOCAL: without the 256 10.5 ms,
-// with it 4.1; on 100,000 pairs 14.4 and 14.1.
-int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total) {
+// with it 4.1; on 100,000 pairs 14.4 and 14.1.  coop: the share of the batch
+// from which a pair takes the block; not with fewer columns than a pass fills
+// in (1000 pairs of 30 x 4000 bases 364 us, on 64 lanes 302).
+int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total, double coop) {
     // least query words for which 64 lanes hold at least 0.85 of the share of 16
     static const std::vector<uint32_t> wide = [] {
         std::vector<uint32_t> v(1024);
@@ -1131,7 +1137,7 @@ int g2_wave_lanes(uint32_t qw, uint32_t tw, uint64_t total) {
     }();
     if (tw <= 32) return 16;
     const double cells = 64.0 * qw * tw;
-    if (tw > 128 && cells > 2.3e-4 * (double)total) return 256;
+    if (tw > 128 && qw >= 16 && cells > coop * (double)total) return 256;
     if (cells > 4e-4 * (double)total) return 64;
     return qw >= wide[std::min<uint32_t>(tw, 1023)] ? 64 : 16;
 }
@@ -1929,11 +1935,19 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         }
         const int policy = g2_get_dispatch();
         if (policy == 3 || (policy == 0 && !(mixed && switched) && g2_wave_pays(op, total, longest, steps))) {
-            for (uint32_t k = 0; k < n && tw > 32; k++) {
-                const int lanes = g2_wave_lanes(g2_regs(hq[k]), g2_regs(ht[k]), total);
-                d.wave_coop += lanes == 256;
-                d.wave64 += lanes == 64;
-            }
+            // more than a device's worth of blocks of four waves: then those
+            // pairs are the batch (1000 x 1100 bases LOCAL, on blocks / 64 lanes:
+            // 1000 pairs 0.67 / 0.79 ms, 2000 1.75 / 1.21, 4000 3.10 / 2.19)
+            double coop = G2_WAVE_COOP;
+            do {
+                d.wave_coop = d.wave64 = 0;
+                for (uint32_t k = 0; k < n && tw > 32; k++) {
+                    const int lanes = g2_wave_lanes(g2_regs(hq[k]), g2_regs(ht[k]), total, coop);
+                    d.wave_coop += lanes == 256;
+                    d.wave64 += lanes == 64;
+                }
+                coop *= 2;
+            } while (d.wave_coop > 4 * g2_cu_count());
         } else {
             d.wave = 0;
         }
