@@ -91,7 +91,7 @@ struct G2Dev {
     // WITH_TB on that path (wavetb.hip): after wave_coop and wave64 as above, the
     // next wave32 and wave16 slots (whole waves of them, or to the end) on 32 and
     // 16 lanes, the rest on 4; tb then holds the waves' checkpoints, wv_at each pair's place in them
-    // and wv_strip (second best) a word per strip of the batch, places claimed from aux[3].
+    // and wv_strip (second best) a word per strip of the batch, places claimed from aux[6..7].
     uint32_t wave32, wave16;
     uint2 *wv_at;
     uint32_t *wv_strip;

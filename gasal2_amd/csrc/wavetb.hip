@@ -82,25 +82,32 @@ __device__ __forceinline__ void wv_pairs(const G2Dev &d, const G2Scores &c, WvSh
     const int32_t P = wv_period(QW, COOP ? 256 : GW), npass = (passes - wv + NW - 1) / NW, strips = ok ? TW : 0;   // npass: this wave's
     const int32_t its = wave_max<GW>(npass > 0 ? npass * P + GW : 0);
     const bool slack = !__any(P < GW + 3);
-    uint32_t it0 = 0;
-    if (lane == 0 && wv == 0) it0 = atomicAdd(&d.aux[4], COOP ? wv_region((uint32_t)passes, P, WV_WAVES) : (uint32_t)its);
-    it0 = __builtin_amdgcn_readfirstlane(it0);
-    // The strips' records of the second best: a place per strip of the batch
-    // (a row of the longest target's strips per pair took n times its length).
-    // k_second_scan finds the pair's first one in wv_sec.
-    uint32_t strip0 = 0;
-    if (SECOND && wv == 0) {
-        const uint32_t own = ok && l == 0 ? (uint32_t)TW : 0u;
+    // The wave's iterations and, for the second best, its pairs' strips, claimed by
+    // one atomic (a second one on the word next to it cost 50 us of 440 on 20,000
+    // pairs, 1250 waves that all start with it).  The strips' records take a place
+    // per strip of the batch (a row of the longest target's strips per pair took n
+    // times its length); k_second_scan finds the pair's first one in wv_sec.
+    uint32_t it0 = 0, strip0 = 0;
+    if (wv == 0) {
+        const uint32_t own = SECOND && ok && l == 0 ? (uint32_t)TW : 0u;
         uint32_t upto = own;
+        if (SECOND) {
 #pragma unroll
-        for (uint32_t off = 1; off < WAVE; off <<= 1) {
-            const uint32_t o = __shfl_up(upto, off);
-            upto += lane >= (int32_t)off ? o : 0u;
+            for (uint32_t off = 1; off < WAVE; off <<= 1) {
+                const uint32_t o = __shfl_up(upto, off);
+                upto += lane >= (int32_t)off ? o : 0u;
+            }
         }
-        uint32_t first = 0;
-        if (lane == WAVE - 1) first = atomicAdd(&d.aux[3], upto);
-        strip0 = __shfl(__shfl(first, WAVE - 1) + upto - own, lane - l);
-        if (own) d.wv_sec[slot] = strip0;
+        unsigned long long got = 0;
+        if (lane == WAVE - 1)
+            got = atomicAdd(reinterpret_cast<unsigned long long *>(d.aux + 6),
+                            (unsigned long long)upto << 32 |
+                                (COOP ? wv_region((uint32_t)passes, P, WV_WAVES) : (uint32_t)its));
+        it0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)got, WAVE - 1);
+        if (SECOND) {
+            strip0 = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(got >> 32), WAVE - 1) + __shfl(upto - own, lane - l);
+            if (own) d.wv_sec[slot] = strip0;
+        }
     }
     if (COOP) {
         if (threadIdx.x == 0) { sh.it0 = it0; sh.strip0 = strip0; }
