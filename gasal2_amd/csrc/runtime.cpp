@@ -1064,18 +1064,24 @@ bool wave_tb_pays(const G2Opts &op, double n, double cells, double longest, doub
     return work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
 }
 
-// Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb), of n
-// paths: their cells on the diagonal and in gaps (GLOBAL's lengths differ by at
-// least those), the longest path's and the most gaps.  A lane takes 0.7 us a cell
-// whatever it is, and hides most of the others' walks behind the longest.  A wave
-// steps over a stretch of matches at once, 38 ps a cell of the sum, and over
-// gaps one by one, 150 ps of the sum and 0.4 us of the longest.  Lanes / waves, us:
-// 100 x 100 bases 10,000 pairs 88 / 56, 60,000 126 / 272; 250 x 250 10,000 201 /
-// 147, 60,000 235 / 621; 1500 x 1500 1000 pairs 1161 / 139; GLOBAL 2000 x 60 1000
-// pairs 1246 / 784, 10,000 1323 / 3387; 30 x 300 1000 231 / 142, 10,000 242 / 374.
-bool wave_walk_pays(double n, double diag, double gaps, double longest, double most_gaps) {
-    const double waves = 15e-6 + std::max(1e-9 * n + 38e-12 * diag + 150e-12 * gaps, 0.4e-6 * most_gaps);
-    return waves < 10e-6 + 0.7e-6 * longest + 11e-12 * (diag + gaps);
+// Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb): the cells
+// of all paths on the diagonal and in gaps (GLOBAL's lengths differ by at least
+// those), and the most of one pair.  A lane takes 1.4 us a cell on the diagonal
+// where the lanes of its wave enter their tiles at different times (half of that
+// where they do not: pairs without indels) and 0.65 in a gap, and hides most of
+// the others' walks behind the longest.  A wave steps over a stretch of matches at
+// once, 0.15 us a cell of the longest path and 55 ps of the sum, and over gaps one
+// by one, 0.4 us and 150 ps.  Lanes / waves, us: 150 x 250 bases LOCAL 10,000 pairs
+// 254 / 119, 20,000 264 / 195, 60,000 284 / 503; GLOBAL 10,000 310 / 232, 20,000
+// 330 / 389; 50-5000 bases LOCAL 20,000 7187 / 750; GLOBAL 2000 x 60 1000 pairs
+// 1246 / 784, 10,000 1323 / 3387; 30 x 300 1000 231 / 142, 10,000 242 / 374.
+struct PathSums {
+    uint64_t diag = 0, gaps = 0;
+    uint32_t most_diag = 0, most_gaps = 0;
+};
+bool wave_walk_pays(const PathSums &p) {
+    const double waves = std::max(55e-12 * p.diag + 150e-12 * p.gaps, 0.15e-6 * p.most_diag + 0.4e-6 * p.most_gaps);
+    return 25e-6 + waves < 10e-6 + 1.4e-6 * p.most_diag + 0.65e-6 * p.most_gaps + 8e-12 * (p.diag + p.gaps);
 }
 
 // Shape buckets as the device sorts by them (k_keys), and a bucket's largest x.
@@ -1668,8 +1674,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         const double scale = n / 4096.0;
         wave_tb = wave_tb_pays(op, n, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
     }
-    uint64_t wave_strips = 0, path_diag = 0, path_gaps = 0, wave_room = 0;
-    uint32_t path_max = 0, gaps_max = 0;
+    uint64_t wave_strips = 0, wave_room = 0;
+    PathSums paths;
     if (wave_tb) {
         uint64_t tiles = 0, longest = 0, work = 0;
         uint32_t least = 0xFFFFFFFFu;
@@ -1681,10 +1687,10 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             work += wave_tb_iters(kq, kt, 4);
             wave_strips += kt;
             const uint32_t diag = std::min(hq[k], ht[k]), gaps = op.algo == LOCAL ? 0 : std::max(hq[k], ht[k]) - diag;
-            path_diag += diag;
-            path_gaps += gaps;
-            path_max = std::max(path_max, diag + gaps);
-            gaps_max = std::max(gaps_max, gaps);
+            paths.diag += diag;
+            paths.gaps += gaps;
+            paths.most_diag = std::max(paths.most_diag, diag);
+            paths.most_gaps = std::max(paths.most_gaps, gaps);
         }
         size_t free_b = 0, total_b = 0;
         wave_tb = least > 0 &&
@@ -1821,7 +1827,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     if (wave_tb) {
         ensure(m->wv_at, m->wv_at_bytes, (size_t)n * 8);
         d.wv_at = m->wv_at;
-        d.wv_walk = wave_walk_pays(n, (double)path_diag, (double)path_gaps, path_max, gaps_max);
+        d.wv_walk = wave_walk_pays(paths);
         if (op.second) {
             ensure(m->wv_strip, m->wv_strip_bytes, (size_t)wave_strips * 4);
             ensure(m->wv_item, m->wv_item_bytes, (size_t)wave_strips * 8);
