@@ -1046,6 +1046,9 @@ uint32_t wave_tb_lanes(uint32_t qw, uint32_t tw, double load, double longest4) {
     return best;
 }
 
+// Pairs of a batch above which some of them are asked first.
+constexpr uint32_t WAVE_SAMPLED = 8192;
+
 // Whether WITH_TB runs there: pairs, padded cells, the longest pair's, and the
 // path's wave-iterations on 4 lanes.  LOCAL: the lane kernels (two pairs a lane) are
 // bound by the longest pair's serial time, part of which other launches on the
@@ -1659,19 +1662,20 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // chunks of 100 to 190 Gcells 8.3 -> 13.4 s with half the memory alone).
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
-    if (wave_tb && n > 65536 && g2_get_dispatch() == 0) {
-        // a large batch that the lane kernels run faster is told by 4096 of its
-        // pairs, with the longest shapes as one pair's (a pass over 1M pairs took
-        // 2 ms of a 24.7 ms step; 300,000 pairs with second best 0.72 ms of host
-        // time a pass where the sample left all but clear cases to the sums, 0.15 so)
+    if (wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
+        // a large batch that the lane kernels run faster is told by a sixteenth of
+        // its pairs, 4096 at most, with the longest shapes as one pair's (a pass
+        // over 1M pairs took 2 ms of a 24.7 ms step; 300,000 pairs with second best
+        // 0.72 ms of host time a pass where the sample left all but clear cases to
+        // the sums, 0.15 so; 60,000 pairs of 16 x 16 bases 0.15 summed, 0.05 sampled)
         uint64_t tiles = 0, work = 0;
-        const uint32_t step = n / 4096;
-        for (uint32_t k = 0; k < 4096; k++) {
+        const uint32_t step = std::max(n / 4096, 16u), count = n / step;
+        for (uint32_t k = 0; k < count; k++) {
             const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
             tiles += (uint64_t)kq * kt;
             work += wave_tb_iters(kq, kt, 4);
         }
-        const double scale = n / 4096.0;
+        const double scale = (double)n / count;
         wave_tb = wave_tb_pays(op, n, 64.0 * scale * tiles, 64.0 * qw * tw, scale * work / 16.0);
     }
     uint64_t wave_strips = 0, wave_room = 0;
@@ -1916,16 +1920,16 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     }
     g2_choose_packed(d, op, sc, eq, et, px.banded);
     if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
-    if (d.wave && !wave_tb && n > 65536 && g2_get_dispatch() == 0) {
+    if (d.wave && !wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
         // as above for the score and start modes (1M pairs GLOBAL 12.7 ms a step, 10.9 of it the device's)
         uint64_t total = 0, steps = 0;
-        const uint32_t step = n / 4096;
-        for (uint32_t k = 0; k < 4096; k++) {
+        const uint32_t step = std::max(n / 4096, 16u), count = n / step;
+        for (uint32_t k = 0; k < count; k++) {
             const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
             total += 64ull * kq * kt;
             steps += g2_wave_steps(kq, kt);
         }
-        const double scale = n / 4096.0;
+        const double scale = (double)n / count;
         if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(scale * steps))) d.wave = 0;
     }
     if (d.wave && !wave_tb) {
