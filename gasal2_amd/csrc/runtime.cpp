@@ -1056,7 +1056,10 @@ constexpr uint32_t WAVE_SAMPLED = 8192;
 // strips included.  100-300 x 100-400 bases with second best, lanes / that path:
 // 30,000 pairs 6.2 / 1.8 ms, 100,000 6.4 / 3.5, 300,000 11.0 / 9.3 alone and 7.9 /
 // 8.2 among other passes, 900,000 19.5 / 26.8; 150 x 250 without: 100,000 pairs
-// 3.0 / 2.0, 300,000 5.7 / 5.0, 1,000,000 15.7 / 17.0.  GLOBAL: its lanes store
+// 3.0 / 2.0, 300,000 5.7 / 5.0, 1,000,000 15.7 / 17.0; a pass with its host time
+// (the plan, 2 ns a pair more): 100 x 100 20,000 0.59 / 0.42, 60,000 0.62 / 0.75, with
+// second best 40,000 0.68 / 0.69, 60,000 0.70 / 0.88; 64 x 64 40,000 0.34 / 0.43; 16
+// x 16 with second best 1000 91 / 125 us.  GLOBAL: its lanes store
 // direction words in 32 bits, whatever the pair's shape, where a wave's pass has
 // five iterations at least and the host plans every pair.  Lanes / that path, a
 // pass with its host time: 100-300 x 100-400 bases 900,000 pairs 26.4 / 23.9 ms;
@@ -1064,7 +1067,22 @@ constexpr uint32_t WAVE_SAMPLED = 8192;
 // 60,000 331 / 514; 16 x 16 1000 109 / 144, 600,000 427 / 2947.
 bool wave_tb_pays(const G2Opts &op, double n, double cells, double longest, double work) {
     if (op.algo == GLOBAL) return 30e-6 + 4e-9 * n + work * 8192.0 / 2.95e12 < 36e-9 * longest + cells / 1.9e12;
-    return work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
+    return 8e-6 + 2e-9 * n + work * 8192.0 / (op.second ? 2.4e12 : 2.95e12) < 20e-9 * longest + cells / 3.6e12;
+}
+
+// Steps of a pair on k_local_fast's one-wave blocks: a pass of 64 strips, column by column.
+uint64_t wf_steps(uint32_t qw, uint32_t tw) { return (uint64_t)((tw + 63) / 64) * (8 * qw + 63); }
+
+// Whether a batch of few pairs LOCAL WITH_TB without second best, which would
+// run there one wave each (1400 at a time), does: by the serial time of the
+// longest pair, the lane's walk of its path included.  That / this path, us:
+// 150 x 150 bases 64 pairs 294 / 175, 16,000 1360 / 494; 8 x 8 10,000 337 / 208;
+// 1000 x 100 1000 700 / 450; 60 x 2000 64 425 / 483, 5000 1245 / 917.
+bool wave_tb_few_pays(uint32_t n, uint32_t qw, uint32_t tw) {
+    uint64_t its = ~0ull;
+    for (uint32_t gw : {4u, 16u, 32u, 64u}) its = std::min(its, wave_tb_iters(qw, tw, gw));
+    if (tw > 128) its = std::min(its, wave_tb_iters(qw, tw, 256) + 195);
+    return 15e-6 + 2.5e-6 * its < (30e-6 + 0.6e-6 * wf_steps(qw, tw) + 5.6e-6 * std::min(qw, tw)) * std::max(1.0, n / 1400.0);
 }
 
 // Whether a wave walks each path (k_wave_walk), or a lane (k_get_tb): the cells
@@ -1662,7 +1680,9 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // chunks of 100 to 190 Gcells 8.3 -> 13.4 s with half the memory alone).
     bool wave_tb = !px.banded && (g2_get_dispatch() == 0 || g2_get_dispatch() == 3) && !(g_wf_user && op.algo == LOCAL && !op.second) &&
                    wave_tb_fits(op, sc, qw, tw, d.fast);
-    if (wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
+    // few pairs LOCAL without second best: the alternative is one wave a pair
+    const bool few_local = op.algo == LOCAL && !op.second && (uint64_t)n <= (uint64_t)g2_cu_count() * WF_FEW_PER_CU_TB;
+    if (wave_tb && !few_local && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
         // a large batch that the lane kernels run faster is told by a sixteenth of
         // its pairs, 4096 at most, with the longest shapes as one pair's (a pass
         // over 1M pairs took 2 ms of a 24.7 ms step; 300,000 pairs with second best
@@ -1682,12 +1702,15 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     PathSums paths;
     if (wave_tb) {
         uint64_t tiles = 0, longest = 0, work = 0;
-        uint32_t least = 0xFFFFFFFFu;
+        uint32_t least = 0xFFFFFFFFu, far = 0;   // far: the longest pair
         for (uint32_t k = 0; k < n; k++) {
             const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
             least = std::min(least, std::min(hq[k], ht[k]));
             tiles += (uint64_t)kq * kt;
-            longest = std::max(longest, (uint64_t)kq * kt);
+            if ((uint64_t)kq * kt > longest) {
+                longest = (uint64_t)kq * kt;
+                far = k;
+            }
             work += wave_tb_iters(kq, kt, 4);
             wave_strips += kt;
             const uint32_t diag = std::min(hq[k], ht[k]), gaps = op.algo == LOCAL ? 0 : std::max(hq[k], ht[k]) - diag;
@@ -1698,7 +1721,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         }
         size_t free_b = 0, total_b = 0;
         wave_tb = least > 0 &&
-                  (g2_get_dispatch() == 3 || wave_tb_pays(op, n, 64.0 * tiles, 64.0 * longest, work / 16.0)) &&
+                  (g2_get_dispatch() == 3 || (few_local ? wave_tb_few_pays(n, g2_regs(hq[far]), g2_regs(ht[far]))
+                                                        : wave_tb_pays(op, n, 64.0 * tiles, 64.0 * longest, work / 16.0))) &&
                   hipMemGetInfo(&free_b, &total_b) == hipSuccess;
         wave_room = std::min(((uint64_t)free_b + m->tb_bytes + m->wv_strip_bytes + m->wv_item_bytes) / 2, g_tb_one_size_max);
         wave_tb = wave_tb && tiles * 64 <= wave_room;
