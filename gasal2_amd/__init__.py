@@ -247,6 +247,8 @@ _SIGS = {
     "gasal2_set_tb_fused": (None, [C.c_int32]),
     "gasal2_set_panels": (None, [C.c_int32]),
     "gasal2_last_paths": (C.c_int32, [C.POINTER(gasal_gpu_storage_t)]),
+    "gasal2_wave_tb_plan": (None, [C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.POINTER(C.c_uint64)]),
+    "gasal2_last_wave_tb": (C.c_int32, [C.POINTER(gasal_gpu_storage_t), C.POINTER(C.c_uint64)]),
     "gasal2_tune_set": (None, [C.c_int32, C.c_int32, C.c_int32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32, C.c_uint32]),
     "gasal2_tune_clear": (None, []),
     "gasal2_tune_count": (C.c_int32, []),
@@ -402,6 +404,15 @@ def set_ksw_extension(w=-1, zdrop=0, end_bonus=5):
     (src/kernels/ksw_kernel_template.h:20,27-29)."""
     lib().gasal2_set_ksw_extension(int(w), int(zdrop))
     lib().gasal2_set_ksw_end_bonus(int(end_bonus))
+
+
+def wave_tb_plan(query_lens, target_lens, n_cu=256):
+    """gasal2_wave_tb_plan: iterations at most, then the pairs on 256, 64, 32, 16
+    and 4 lanes (on the host alone)."""
+    q, t = (np.ascontiguousarray(a, dtype=np.uint32) for a in (query_lens, target_lens))
+    out = (C.c_uint64 * 6)()
+    lib().gasal2_wave_tb_plan(q.ctypes.data, t.ctypes.data, len(q), n_cu, out)
+    return list(out)
 
 
 def set_n_penalty(penalty):
@@ -779,8 +790,15 @@ class Aligner:
 
     def last_paths(self):
         """gasal2_last_paths: bit 0 packed 16-bit lane kernel, bit 1 one-wave
-        blocks, bit 2 checkpointed traceback."""
+        blocks, bit 2 checkpointed traceback, bit 3 packed one-wave path, bit 4
+        KSW in packed strips, bit 5 BANDED in packed halves."""
         return int(self._L.gasal2_last_paths(C.byref(self.s)))
+
+    def last_wave_tb(self):
+        """gasal2_last_wave_tb: iterations planned and claimed, then the pairs on
+        256, 64, 32, 16 and 4 lanes; None when the last batch took another path."""
+        out = (C.c_uint64 * 7)()
+        return list(out) if self._L.gasal2_last_wave_tb(C.byref(self.s), out) == 0 else None
 
 
 class PairSet:

@@ -178,6 +178,8 @@ struct Impl {
     bool main_valid = false;
     bool prepped = false;            // resident batch packed/reverse-complemented by gasal2_prep_resident
     int32_t last_paths = 0;          // gasal2_last_paths of the last launched batch
+    uint64_t wave_plan = 0;          // iterations planned for the last batch on the packed one-wave traceback path
+    uint32_t last_wave[5] = {};      // and its pairs on 256, 64, 32, 16 and 4 lanes (all 0: another path)
 };
 
 Impl *impl_of(gasal_gpu_storage_t *s) {
@@ -1488,7 +1490,8 @@ G2Opts opts_of(const Parameters *p, const gasal_gpu_storage_t *s) {
 // iterations its waves can claim together: the batch's shapes in the device's
 // sorted order (k_keys), each bucket at its largest shape, every wave at its
 // longest pair's.
-uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht, uint32_t n, uint32_t qw, uint32_t tw) {
+uint64_t wave_tb_plan(std::vector<uint32_t> &keys, std::vector<uint32_t> &khist, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
+                      uint32_t n, uint32_t qw, uint32_t tw, uint32_t n_cu) {
     std::vector<std::pair<uint32_t, uint32_t>> runs;   // key, pairs, in descending key order
     auto key_of = [&](uint32_t k) -> uint32_t {
         const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
@@ -1496,25 +1499,25 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
         return (lng ? 0x10000u : 0u) | (shape8(kq) << 8) | shape8(kt);
     };
     if (n <= 8192) {
-        m->h_keys.resize(n);
-        for (uint32_t k = 0; k < n; k++) m->h_keys[k] = key_of(k);
-        std::sort(m->h_keys.begin(), m->h_keys.end(), std::greater<uint32_t>());
+        keys.resize(n);
+        for (uint32_t k = 0; k < n; k++) keys[k] = key_of(k);
+        std::sort(keys.begin(), keys.end(), std::greater<uint32_t>());
         for (uint32_t k = 0; k < n; k++) {
-            if (k == 0 || m->h_keys[k] != m->h_keys[k - 1]) runs.push_back({m->h_keys[k], 0});
+            if (k == 0 || keys[k] != keys[k - 1]) runs.push_back({keys[k], 0});
             runs.back().second++;
         }
     } else {
         // counters stay zero between batches; only rows that hold pairs are read
-        m->h_khist.resize(G2_SHAPE_BUCKETS, 0u);
+        khist.resize(G2_SHAPE_BUCKETS, 0u);
         bool rows[G2_SHAPE_ROWS] = {};
         for (uint32_t k = 0; k < n; k++) {
             const uint32_t key = key_of(k);
-            m->h_khist[key]++;
+            khist[key]++;
             rows[key >> 8] = true;
         }
         for (uint32_t row = G2_SHAPE_ROWS; row-- > 0;)
             for (uint32_t c = 256; rows[row] && c-- > 0;)
-                if (uint32_t &v = m->h_khist[row * 256 + c]) {
+                if (uint32_t &v = khist[row * 256 + c]) {
                     runs.push_back({row * 256 + c, v});
                     v = 0;
                 }
@@ -1527,7 +1530,7 @@ uint64_t wave_tb_plan(Impl *m, G2Dev &d, const uint32_t *hq, const uint32_t *ht,
         work += r.second * its / 16.0;
         longest4 = std::max(longest4, its);
     }
-    const double load = work / (4.0 * std::max(g2_cu_count(), 1u));
+    const double load = work / (4.0 * std::max(n_cu, 1u));
     uint32_t n256 = 0, n64 = 0, n32 = 0, n16 = 0;
     for (const auto &r : runs) {
         const uint32_t lanes = wave_tb_lanes(q_of(r.first), t_of(r.first), load, longest4);
@@ -1784,7 +1787,8 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     }
     uint64_t wave_bytes = 0;
     if (wave_tb) {
-        wave_bytes = wave_tb_plan(m, d, hq, ht, n, qw, tw) * 8192;
+        m->wave_plan = wave_tb_plan(m->h_keys, m->h_khist, d, hq, ht, n, qw, tw, g2_cu_count());
+        wave_bytes = m->wave_plan * 8192;
         // with the allocator's slack (ensure)
         const uint64_t need = wave_bytes + (op.second ? wave_strips * 12 : 0);
         if (need + need / 8 > wave_room || wave_strips > 0xFFFFFFFFull) {
@@ -2018,7 +2022,12 @@ void upload_async(gasal_gpu_storage_t *s, uint32_t n, Parameters *params) {
 // trigger a new capture.  The program holds kernels only (no memset or copy
 // nodes).  Timed runs (per-stage events) launch eagerly.
 hipError_t launch_program(Impl *m, const G2Scores &sc, const G2Opts &op, const G2Dev &d, hipStream_t st) {
-    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16 || d.band_pk) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh || (d.wave && op.start == WITH_TB) ? 4 : 0);
+    m->last_paths = ((d.wave || d.pk16 || d.pk2 || d.pk16g || d.pk16s || d.ksw16 || d.band_pk) ? 1 : 0) | (d.wf_blocks || d.wave ? 2 : 0) | (d.tbh || (d.wave && op.start == WITH_TB) ? 4 : 0) |
+                    (d.wave ? 8 : 0) | (d.ksw_pk ? 16 : 0) | (d.band_pk ? 32 : 0);
+    const bool wave_tb = d.wave && op.start == WITH_TB;
+    const uint32_t narrow = d.n - d.wave_coop - d.wave64 - d.wave32 - d.wave16;
+    const uint32_t lanes[5] = {d.wave_coop, d.wave64, d.wave32, d.wave16, narrow};
+    for (int k = 0; k < 5; k++) m->last_wave[k] = wave_tb ? lanes[k] : 0;
     if (!g_graph_mode || m->tm.enabled) return g2_run(sc, op, d, st, &m->tm);
     const bool same = m->g_valid && memcmp(&m->g_dev, &d, sizeof(d)) == 0 && memcmp(&m->g_sc, &sc, sizeof(sc)) == 0 &&
                       memcmp(&m->g_op, &op, sizeof(op)) == 0;
@@ -2195,6 +2204,41 @@ extern "C" float gasal2_stage_ms(gasal_gpu_storage_t *s, int32_t stage) {
     if (hipEventSynchronize(m->tm.ev[b[stage]]) != hipSuccess) return -1.0f;
     if (hipEventElapsedTime(&ms, m->tm.ev[a[stage]], m->tm.ev[b[stage]]) != hipSuccess) return -1.0f;
     return ms;
+}
+
+// The packed one-wave traceback path's plan for pairs of these lengths (at least
+// one base each), on the host alone.
+extern "C" void gasal2_wave_tb_plan(const uint32_t *query_lens, const uint32_t *target_lens, uint32_t n, uint32_t n_cu,
+                                    uint64_t *out) {
+    uint32_t mq = 0, mt = 0;
+    for (uint32_t k = 0; k < n; k++) {
+        mq = std::max(mq, query_lens[k]);
+        mt = std::max(mt, target_lens[k]);
+    }
+    G2Dev d;
+    memset(&d, 0, sizeof(d));
+    std::vector<uint32_t> keys, khist;
+    out[0] = n ? wave_tb_plan(keys, khist, d, query_lens, target_lens, n, g2_regs(mq), g2_regs(mt), n_cu) : 0;
+    out[1] = d.wave_coop;
+    out[2] = d.wave64;
+    out[3] = d.wave32;
+    out[4] = d.wave16;
+    out[5] = n - d.wave_coop - d.wave64 - d.wave32 - d.wave16;
+}
+
+extern "C" int32_t gasal2_last_wave_tb(gasal_gpu_storage_t *s, uint64_t *out) {
+    if (!s || !s->impl) return -1;
+    Impl *m = impl_of(s);
+    uint64_t pairs = 0;
+    for (int k = 0; k < 5; k++) pairs += out[2 + k] = m->last_wave[k];
+    if (!pairs) return -1;
+    uint32_t claimed = 0;
+    if (hipStreamSynchronize(s->str) != hipSuccess ||
+        hipMemcpy(&claimed, m->aux + 6, sizeof(claimed), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    out[0] = m->wave_plan;
+    out[1] = claimed;
+    return 0;
 }
 
 // ------------------------------------------------ banded runs and fallback ---

@@ -218,8 +218,22 @@ void gasal2_set_panels(int32_t on);
 /* Which kernel paths the storage's last batch took (no counterpart in the
  * reference; for measurement): bit 0 a packed 16-bit kernel on the
  * one-lane-per-pair path (or KSW's packed row), bit 1 one-wave-per-pair
- * blocks, bit 2 checkpointed traceback (lane path or packed one-wave path). */
+ * blocks, bit 2 checkpointed traceback (lane path or packed one-wave path),
+ * bit 3 the packed one-wave path, bit 4 KSW in packed strips, bit 5 BANDED in
+ * packed halves (the last three while the batch's nibbles allow score tables). */
 int32_t gasal2_last_paths(gasal_gpu_storage_t *storage);
+
+/* WITH_TB on the packed one-wave path (no counterpart in the reference; for
+ * measurement and to size gasal2_set_tile_budget).  Its checkpoints are a log of
+ * 8 KiB iterations.  gasal2_wave_tb_plan: for pairs of these lengths on a device
+ * of n_cu compute units, out[0] the iterations at most, out[1..5] the pairs on
+ * 256, 64, 32, 16 and 4 lanes; it runs on the host alone.  gasal2_last_wave_tb:
+ * of the storage's last batch, out[0] the iterations planned, out[1] those its
+ * waves claimed (it waits for the batch), out[2..6] the pairs as above; -1 when the
+ * batch took another path. */
+void gasal2_wave_tb_plan(const uint32_t *query_lens, const uint32_t *target_lens, uint32_t n, uint32_t n_cu,
+                         uint64_t *out);
+int32_t gasal2_last_wave_tb(gasal_gpu_storage_t *storage, uint64_t *out);
 
 /* Graph mode (default on): each storage captures its device program (pack,
  * reverse/complement, shape ordering, DP, traceback) into a HIP graph the first
