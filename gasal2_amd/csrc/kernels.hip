@@ -2567,7 +2567,8 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     uint32_t bflag = 0;
     if (band && (d.band_flags[pr] & 8u)) { d.n_ops[pr] = 0; return; }
     // GLOBAL words are always in the sign-bit format (k_global)
-    const bool lanefast = d.fast && d.enc_ok && census_fast(census);
+    // the lane path ran with score tables: one pair a lane, or two
+    const bool lanefast = d.fast && (d.enc_ok || d.pk2) && census_fast(census);
     const bool fastfmt = !LOCALT || band || wfp || lanefast;
     // lane-path tiles of k_local_fast<.., CK> are recomputed from checkpoints
     const bool ck = LOCALT && !band && !wfp && !WV && lanefast && d.tbh != nullptr;
