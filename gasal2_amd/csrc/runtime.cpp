@@ -981,6 +981,12 @@ extern "C" void gasal_gpu_mem_free(gasal_gpu_storage_t *gpu_storage, Parameters 
 // Packed and table kernels for a batch: the choices depend only on the
 // mode, the scores and the largest shape the lane path runs (eq query words,
 // et target words); shared by the storage path and gasal2_aln_noalloc.
+// Best score a cell can add: a negative mismatch or N penalty counts as the match
+// does.
+int64_t best_cell(const G2Scores &sc) {
+    return std::max<int64_t>({sc.match, -(int64_t)sc.mismatch, sc.has_np ? -(int64_t)sc.np : 0, 0});
+}
+
 // Whether the packed one-wave path (wave.hip) can run a batch whose largest
 // pair has qw query and tw target words: its G2Dev::wave value, 0 when a value
 // could leave 16 bits.  LOCAL holds E and F at or above 0, so only H <= the
@@ -994,8 +1000,7 @@ uint32_t g2_wave_fits(const G2Opts &op, const G2Scores &sc, uint32_t qw, uint32_
     if (op.algo != LOCAL && op.algo != GLOBAL && op.algo != SEMI_GLOBAL) return 0;
     if (sc.gapo < 0 || sc.gape < 0 || sc.gapo > 16000 || sc.gape > 255) return 0;
     if (8ull * qw + 256 > 65535) return 0;   // steps of a pass are held in 16 bits
-    const int64_t nval = sc.has_np ? -sc.np : 0;
-    const int64_t up = std::max<int64_t>({sc.match, -(int64_t)sc.mismatch, nval, 0});
+    const int64_t nval = sc.has_np ? -sc.np : 0, up = best_cell(sc);
     const int64_t down = std::max<int64_t>({-(int64_t)sc.match, sc.mismatch, -nval, 0});
     const int64_t hmax = up * 8 * std::min<int64_t>(qw, tw);
     if (op.algo == LOCAL) return hmax <= 8191 ? 1 : (hmax <= 32000 ? 2 : 0);
@@ -1175,24 +1180,24 @@ void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t e
     auto bl = [](uint64_t v) { int b = 0; while (v) { b++; v >>= 1; } return b; };
     // Packed 16-bit LOCAL (score and ends; WITH_START then runs the int32
     // reverse pass on the packed forward's end): every value of the pairs the lane
-    // path runs fits int16 -- H <= match * min(8 eq, 8 et); E, F >= -(mismatch,
+    // path runs fits int16 -- H <= best cell * min(8 eq, 8 et); E, F >= -(mismatch,
     // N penalty) - open - 9 extend -- and the policy allows it.
     d.pk16 = 0;
     if (d.fast && op.algo == LOCAL && (op.start == WITHOUT_START || op.start == WITH_START) && !op.second && g_pk16_mode) {
-        const int64_t hmax = (int64_t)std::max(sc.match, 0) * std::min<int64_t>(8ll * eq, 8ll * et);
+        const int64_t hmax = best_cell(sc) * std::min<int64_t>(8ll * eq, 8ll * et);
         const int64_t lowest = -(int64_t)std::max(sc.mismatch, sc.has_np ? sc.np : 0) - sc.gapoe - 9ll * sc.gape - 8;
         if (hmax <= 32000 && lowest >= -32000) d.pk16 = 1;
     }
     // Two pairs per lane in packed 16-bit halves (k_local_pk2): LOCAL with
     // second best or the checkpointed traceback (policy 2: every LOCAL mode).
-    // Cells are ranked as h * 8 + (7 - row) in 16 bits, so H <= match *
+    // Cells are ranked as h * 8 + (7 - row) in 16 bits, so H <= best cell *
     // min(8 eq, 8 et) must stay <= 4095; column indices i * 8 eq + t must fit
     // 16 bits; E and F stay above -32000 as for pk16.
     d.pk2 = 0;
     if (d.fast && op.algo == LOCAL && !banded && g_pk16_mode) {
         const bool tb_ok = op.start != WITH_TB || (d.tbh && !d.tb_fused);
         const bool want = g_pk16_mode == 2 || op.second || op.start == WITH_TB;
-        const int64_t hmax = (int64_t)std::max(sc.match, 0) * std::min<int64_t>(8ll * eq, 8ll * et);
+        const int64_t hmax = best_cell(sc) * std::min<int64_t>(8ll * eq, 8ll * et);
         const int64_t lowest = -(int64_t)std::max(sc.mismatch, sc.has_np ? sc.np : 0) - sc.gapoe - 9ll * sc.gape - 8;
         if (tb_ok && want && hmax <= 4095 && lowest >= -32000 && (uint64_t)et * 8u * eq <= 65535u) {
             d.pk2 = 1;
@@ -1207,7 +1212,7 @@ void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t e
     if (d.fast && op.algo == GLOBAL && op.start != WITH_TB && g_pk16_mode && sc.gape <= 255) {
         const int64_t pen = std::max<int64_t>(std::max(sc.mismatch, sc.has_np ? sc.np : 0), 0);
         const int64_t sh = 8ll * std::min(eq, et), lg = 8ll * ((int64_t)eq + et);
-        const int64_t bound = (pen + std::max(sc.match, 0)) * sh + 2ll * sc.gapoe + (int64_t)sc.gape * lg + pen;
+        const int64_t bound = (pen + best_cell(sc)) * sh + 2ll * sc.gapoe + (int64_t)sc.gape * lg + pen;
         if (bound <= 16000) d.pk16g = 1;
     }
     // Packed 16-bit SEMI_GLOBAL: the same bound (head gaps as GLOBAL's
@@ -1217,7 +1222,7 @@ void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t e
         g_pk16_mode && sc.gape <= 255) {
         const int64_t pen = std::max<int64_t>(std::max(sc.mismatch, sc.has_np ? sc.np : 0), 0);
         const int64_t sh = 8ll * std::min(eq, et), lg = 8ll * ((int64_t)eq + et);
-        const int64_t bound = (pen + std::max(sc.match, 0)) * sh + 2ll * sc.gapoe + (int64_t)sc.gape * lg + pen;
+        const int64_t bound = (pen + best_cell(sc)) * sh + 2ll * sc.gapoe + (int64_t)sc.gape * lg + pen;
         if (bound <= 16000) d.pk16s = 1;
     }
     // LOCAL lane-per-pair score-table kernel: position encoding
@@ -1225,7 +1230,7 @@ void g2_choose_packed(G2Dev &d, const G2Opts &op, const G2Scores &sc, uint32_t e
     // (all pairs, or those the one-wave path leaves).
     if (d.fast && op.algo == LOCAL) {
         const int cb = std::max(1, bl(8ull * eq - 1)), sbits = std::max(1, bl(et - 1));
-        const uint64_t maxh = (uint64_t)std::max(sc.match, 0) * std::min<uint64_t>(8ull * eq, 8ull * et);
+        const uint64_t maxh = (uint64_t)best_cell(sc) * std::min<uint64_t>(8ull * eq, 8ull * et);
         const int hb = bl(maxh) + 1;
         const int S = 3 + cb + sbits;
         if (S + hb <= 31) {
@@ -1660,8 +1665,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     uint64_t ksw_hmax = ~0ull;
     if (op.algo == KSW && s->host_seed_scores && !px.sub) {   // every KSW value lies in [0, h0 + best score of a cell * min(Lq, Lt)]
         uint64_t hmax = 0;
-        // a negative mismatch or N penalty adds too
-        const uint64_t up = (uint64_t)std::max({g_scores.match, -g_scores.mismatch, g_scores.has_np ? -g_scores.np : 0, 0});
+        const uint64_t up = (uint64_t)best_cell(g_scores);
         for (uint32_t k = 0; k < n; k++)
             hmax = std::max<uint64_t>(hmax, (uint64_t)s->host_seed_scores[k] + up * std::min(hq[k], ht[k]));
         if (hmax <= 65535 && g_pk16_mode) d.ksw16 = 1;
@@ -1819,7 +1823,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             const bool room = g_tb_ckpt == 2 && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
                               wtot * 64 <= ((uint64_t)free_b + m->wf_tb_bytes) / 10 * 8;
             const bool wck = g_tb_ckpt == 2 && room &&
-                             (uint64_t)std::max(g_scores.match, 0) * 8u * std::min(lqw, ltw) <= 32767u &&
+                             (uint64_t)best_cell(g_scores) * 8u * std::min(lqw, ltw) <= 32767u &&
                              (uint64_t)g_scores.gapoe +
                                      (uint64_t)std::max(std::max(g_scores.mismatch, g_scores.has_np ? g_scores.np : 0), 0) <=
                                  32767u;
@@ -1834,7 +1838,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
     // lies in [-open, H], and ranked cells need H <= 8191; steps are held in 16
     // bits.
     if (op.algo == BANDED && d.fast && g_pk16_mode && sc.gape >= 0 && sc.gape <= 16000 && sc.gapoe >= 0 && sc.gapoe <= 16000 &&
-        (int64_t)std::max({sc.match, -sc.mismatch, sc.has_np ? -sc.np : 0, 0}) * 8 * std::min(qw, tw) <= 8191 &&
+        best_cell(sc) * 8 * std::min(qw, tw) <= 8191 &&
         8ull * qw + 8 <= 65535)
         d.band_pk = 1;
     // KSW in packed strips: the reference's form (no band, no z-drop), ranked
@@ -1875,9 +1879,9 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         const uint64_t one_size = lgroups * et * (8 * (uint64_t)eq) * 64 * 4;
         // Checkpointed traceback: two regions of the tile layout (left column
         // states, strip bottom rows) instead of direction words.  Stored
-        // states are 16-bit, so H must fit: H <= match * min(Lq, Lt).
+        // states are 16-bit, so H must fit: H <= best cell * min(Lq, Lt).
         const bool ck = g_tb_ckpt && !wave_tb && op.algo == LOCAL && op.start == WITH_TB && d.fast &&
-                        (uint64_t)std::max(sc.match, 0) * 8u * std::min(eq, et) <= 32767u &&
+                        (uint64_t)best_cell(sc) * 8u * std::min(eq, et) <= 32767u &&
                         (uint64_t)sc.gapoe + (uint64_t)std::max(std::max(sc.mismatch, sc.has_np ? sc.np : 0), 0) <= 32767u;
         const uint64_t nreg = ck ? 2 : 1;
         // One region size for all groups while it is within the budget and
