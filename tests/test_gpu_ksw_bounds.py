@@ -71,3 +71,23 @@ def test_memory_of_one_long_target():
     ref = O.align(b, g.KSW)
     for f in FIELDS:
         assert np.array_equal(got[f], ref[f]), f
+
+
+@pytest.mark.parametrize("scores", [(1, 4, 6, 1), (1, 4, 2, 8), (2, 3, 0, 3), (3, 2, 5, 0)])
+@pytest.mark.parametrize("top_seed", [1, 40, 900])
+def test_first_rows_of_long_queries(scores, top_seed):
+    """Queries longer than the columns a path can reach in the first sixteen rows,
+    related from the start, later or not at all."""
+    rng = np.random.default_rng(9400 + top_seed)
+    qs, ts = [], []
+    for k in range(150):
+        q = rng.choice(list(b"ACGT"), int(rng.integers(200, 700))).astype(np.uint8)
+        t = rng.choice(list(b"ACGT"), int(rng.integers(20, 300))).astype(np.uint8)
+        o = int(rng.integers(0, 60)) if k % 3 else 0
+        m = max(min(len(q) - o, len(t)), 0)
+        if k % 4:
+            t[:m] = q[o:o + m]
+            t[rng.random(len(t)) < 0.04] = ord("N")
+        qs.append(q.tobytes())
+        ts.append(t.tobytes())
+    check(g.make_batch(qs, ts, seeds=rng.integers(0, top_seed, 150).astype(np.uint32)), scores, 1)
