@@ -1847,9 +1847,53 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         sc.gape >= 0 && sc.gape <= 255 && sc.gapoe >= 1 && sc.gapoe <= 16000 && op.ksw_eb <= sc.gapoe &&
         8ull * qw + 8 <= 65535)
         d.ksw_pk = 1;
+    if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
+    if (d.wave && !wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
+        // as above for the score and start modes (1M pairs GLOBAL 12.7 ms a step, 10.9 of it the device's)
+        uint64_t total = 0, steps = 0;
+        const uint32_t step = std::max(n / 4096, 16u), count = n / step;
+        for (uint32_t k = 0; k < count; k++) {
+            const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
+            total += 64ull * kq * kt;
+            steps += g2_wave_steps(kq, kt);
+        }
+        const double scale = (double)n / count;
+        if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(scale * steps))) d.wave = 0;
+    }
+    if (d.wave && !wave_tb) {
+        // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
+        const bool mixed = op.algo == LOCAL && op.start == WITHOUT_START;
+        uint64_t total = 0, longest = 0, steps = 0;
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
+            const uint64_t cells = 64ull * kq * kt;
+            total += cells;
+            steps += g2_wave_steps(kq, kt);
+            if (!mixed || kt < g_wf_min_tw || cells < g_wf_min_cells) longest = std::max(longest, cells);
+        }
+        const int policy = g2_get_dispatch();
+        if (policy == 3 || (policy == 0 && !(mixed && switched) && g2_wave_pays(op, total, longest, steps))) {
+            // more than a device's worth of blocks of four waves: then those
+            // pairs are the batch (1000 x 1100 bases LOCAL, on blocks / 64 lanes:
+            // 1000 pairs 0.67 / 0.79 ms, 2000 1.75 / 1.21, 4000 3.10 / 2.19)
+            double coop = G2_WAVE_COOP;
+            do {
+                d.wave_coop = d.wave64 = 0;
+                for (uint32_t k = 0; k < n && tw > 32; k++) {
+                    const int lanes = g2_wave_lanes(g2_regs(hq[k]), g2_regs(ht[k]), total, coop);
+                    d.wave_coop += lanes == 256;
+                    d.wave64 += lanes == 64;
+                }
+                coop *= 2;
+            } while (d.wave_coop > 4 * g2_cu_count());
+        } else {
+            d.wave = 0;
+        }
+    }
     // Transposed sequence panels for the fast LOCAL lane path (k_panel):
-    // groups after the long pairs, eq query words and et target words each.
-    if (g_panels && d.fast && op.algo == LOCAL && !px.banded && !wave_tb && n > nlong) {
+    // groups after the long pairs, eq query words and et target words each.  The
+    // packed one-wave path reads its pairs' own words.
+    if (g_panels && d.fast && op.algo == LOCAL && !px.banded && !d.wave && n > nlong) {
         const uint64_t lgroups = ((uint64_t)(n - nlong) + 63) / 64;
         ensure(m->qpan, m->qpan_bytes, (size_t)(lgroups * eq * 256) + 256);
         ensure(m->tpan, m->tpan_bytes, (size_t)(lgroups * et * 256) + 256);
@@ -1951,49 +1995,6 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         s->packed_tb_matrix_size = m->tb_bytes / 16;
     }
     g2_choose_packed(d, op, sc, eq, et, px.banded);
-    if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
-    if (d.wave && !wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
-        // as above for the score and start modes (1M pairs GLOBAL 12.7 ms a step, 10.9 of it the device's)
-        uint64_t total = 0, steps = 0;
-        const uint32_t step = std::max(n / 4096, 16u), count = n / step;
-        for (uint32_t k = 0; k < count; k++) {
-            const uint32_t kq = g2_regs(hq[k * step]), kt = g2_regs(ht[k * step]);
-            total += 64ull * kq * kt;
-            steps += g2_wave_steps(kq, kt);
-        }
-        const double scale = (double)n / count;
-        if (!g2_wave_pays(op, (uint64_t)(scale * total), 64ull * qw * tw, (uint64_t)(scale * steps))) d.wave = 0;
-    }
-    if (d.wave && !wave_tb) {
-        // pairs of this size leave the lane kernels for k_local_fast's one-wave blocks
-        const bool mixed = op.algo == LOCAL && op.start == WITHOUT_START;
-        uint64_t total = 0, longest = 0, steps = 0;
-        for (uint32_t k = 0; k < n; k++) {
-            const uint32_t kq = g2_regs(hq[k]), kt = g2_regs(ht[k]);
-            const uint64_t cells = 64ull * kq * kt;
-            total += cells;
-            steps += g2_wave_steps(kq, kt);
-            if (!mixed || kt < g_wf_min_tw || cells < g_wf_min_cells) longest = std::max(longest, cells);
-        }
-        const int policy = g2_get_dispatch();
-        if (policy == 3 || (policy == 0 && !(mixed && switched) && g2_wave_pays(op, total, longest, steps))) {
-            // more than a device's worth of blocks of four waves: then those
-            // pairs are the batch (1000 x 1100 bases LOCAL, on blocks / 64 lanes:
-            // 1000 pairs 0.67 / 0.79 ms, 2000 1.75 / 1.21, 4000 3.10 / 2.19)
-            double coop = G2_WAVE_COOP;
-            do {
-                d.wave_coop = d.wave64 = 0;
-                for (uint32_t k = 0; k < n && tw > 32; k++) {
-                    const int lanes = g2_wave_lanes(g2_regs(hq[k]), g2_regs(ht[k]), total, coop);
-                    d.wave_coop += lanes == 256;
-                    d.wave64 += lanes == 64;
-                }
-                coop *= 2;
-            } while (d.wave_coop > 4 * g2_cu_count());
-        } else {
-            d.wave = 0;
-        }
-    }
 }
 
 G2Scores scores_now() { return g_scores; }

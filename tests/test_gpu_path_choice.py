@@ -1,6 +1,8 @@
 """Which kernels the automatic policy takes where one side clearly wins, by the
 bits of gasal2_last_paths, the results equal to those of the other side."""
+import numpy as np
 import pytest
+import torch
 
 import gasal2_amd as g
 from parity import assert_same, fields
@@ -18,3 +20,27 @@ def test_global_tb_of_short_pairs_on_lanes(n, length, packed):
     (auto, paths), (other, _) = run(b, g.GLOBAL, False, 0, sample), run(b, g.GLOBAL, False, 2 if packed else 3, sample)
     assert bool(paths & 4) == packed
     assert_same(auto, other, fields(g.GLOBAL, g.WITH_TB, False) + ["n_ops", "cigars"], "other side")
+
+
+@pytest.mark.parametrize("start", [g.WITHOUT_START, g.WITH_START])
+def test_packed_scores_take_no_panels(start):
+    """The lane kernels' sequence panels are a row of the longest target's words for
+    every pair (2 GB here); the packed path reads its pairs' own words."""
+    rng = np.random.default_rng(7600)
+    t = rng.choice(list(b"ACGT"), 100_000).astype(np.uint8)
+    qs = [t[o:o + 40].tobytes() for o in rng.integers(0, 1000, 40_000)]
+    b = g.make_batch(qs, qs[:-1] + [t.tobytes()])
+    g.lib().gasal2_set_dispatch(3)
+    a = g.Aligner(g.Parameters(algo=g.LOCAL, start_pos=start), 40, 100_000, b.n)
+    try:
+        a.load(b, per_pair=False)
+        free = torch.cuda.mem_get_info()[0]
+        a.run_resident()
+        a.sync()
+        took = free - torch.cuda.mem_get_info()[0]
+        assert a.last_paths() & 8
+        assert (a.download()["score"][:-1] == 40).all()
+    finally:
+        g.lib().gasal2_set_dispatch(0)
+        a.close()
+    assert took < 3e8, took
