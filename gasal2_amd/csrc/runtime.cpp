@@ -1848,7 +1848,13 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
         8ull * qw + 8 <= 65535)
         d.ksw_pk = 1;
     if (!px.banded) d.wave = wave_tb ? 1 : g2_wave_fits(op, sc, qw, tw, d.fast);
-    if (d.wave && !wave_tb && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
+    // Few pairs LOCAL, scores and ends: the other side is one wave a pair
+    // (k_local_fast), which this path beats throughout.  That / this path, us: 8 x 8
+    // bases 1 pair 95 / 41, 16 x 16 32,000 597 / 221, 300 x 30 20,000 1415 / 520, 2000 x
+    // 2000 300 2569 / 1238, 5000 x 5000 1 15,160 / 3371, 50-5000 bases 10,000 15,396 / 3551.
+    const bool few_scores = op.algo == LOCAL && op.start == WITHOUT_START && !switched &&
+                            (uint64_t)n <= (uint64_t)g2_cu_count() * WF_FEW_PER_CU;
+    if (d.wave && !wave_tb && !few_scores && n > WAVE_SAMPLED && g2_get_dispatch() == 0) {
         // as above for the score and start modes (1M pairs GLOBAL 12.7 ms a step, 10.9 of it the device's)
         uint64_t total = 0, steps = 0;
         const uint32_t step = std::max(n / 4096, 16u), count = n / step;
@@ -1872,7 +1878,7 @@ void prepare(gasal_gpu_storage_t *s, uint32_t qb, uint32_t tb, uint32_t n, const
             if (!mixed || kt < g_wf_min_tw || cells < g_wf_min_cells) longest = std::max(longest, cells);
         }
         const int policy = g2_get_dispatch();
-        if (policy == 3 || (policy == 0 && !(mixed && switched) && g2_wave_pays(op, total, longest, steps))) {
+        if (policy == 3 || (policy == 0 && !(mixed && switched) && (few_scores || g2_wave_pays(op, total, longest, steps)))) {
             // more than a device's worth of blocks of four waves: then those
             // pairs are the batch (1000 x 1100 bases LOCAL, on blocks / 64 lanes:
             // 1000 pairs 0.67 / 0.79 ms, 2000 1.75 / 1.21, 4000 3.10 / 2.19)

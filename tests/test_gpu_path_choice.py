@@ -44,3 +44,20 @@ def test_packed_scores_take_no_panels(start):
         g.lib().gasal2_set_dispatch(0)
         a.close()
     assert took < 3e8, took
+
+
+@pytest.mark.parametrize("n,lq,lt", [(1, 8, 8), (3000, 16, 16), (2000, 300, 30), (40, 1500, 1500)])
+def test_few_scores_on_the_packed_path(n, lq, lt):
+    """Few pairs LOCAL, scores and ends: the one-wave blocks, the other side, are slower at every shape."""
+    b = related(7700 + n, n, (lq, lq), (lt, lt))
+    out = []
+    for policy in (0, 2):
+        g.lib().gasal2_set_dispatch(policy)
+        a = g.Aligner(g.Parameters(algo=g.LOCAL), lq, lt, n)
+        try:
+            out.append(a.run(b, per_pair=False))
+            assert bool(a.last_paths() & 8) == (policy == 0)
+        finally:
+            g.lib().gasal2_set_dispatch(0)
+            a.close()
+    assert_same(out[0], out[1], fields(g.LOCAL, g.WITHOUT_START, False), "lane path")
