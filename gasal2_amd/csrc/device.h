@@ -127,11 +127,10 @@ __device__ __forceinline__ uint32_t rev_word(const uint32_t *W, int32_t len, int
     return nib_reverse(win);
 }
 
-// Recomputes one 8x8 tile's direction words (k_local_fast's sign-bit format)
-// from the checkpoints k_local_fast<.., CK> stored: the previous strip's
-// bottom row above the tile and the tile's left column state.  Same
-// recurrences and score tables (lut: the strip's eight rows, as k_local_fast
-// builds them), so the same words.
+// Recomputes one 8x8 tile's direction words from the checkpoints that the
+// lane kernels (k_local_fast<.., CK>, k_local_pk2) or the packed one-wave path
+// stored: the previous strip's bottom row above the tile and the tile's left
+// column state.  Same recurrences and score tables (lut: the strip's eight rows).
 // top: the row above, entry kk = (H at column kk - 1, E at column kk), so the
 // entry left of the tile's first column (the corner) comes with it; zero above
 // strip 0.  left: the left column state; lut: the strip's score tables (the

@@ -84,7 +84,7 @@ struct G2Dev {
     uint32_t enc_cm, enc_sm;         // column / strip field masks
     // packed one-wave path (wave.hip): every pair on a group of lanes, the
     // first wave_coop sorted slots on a block of four waves, the next wave64
-    // on 64 lanes, the rest on 16.  0: off, 1: cells
+    // on 64 lanes, the rest on 16 (WITH_TB: below).  0: off, 1: cells
     // ranked with their row (LOCAL: H <= 8191), 2: H alone.  When the census
     // refuses the score tables the lane kernels run the batch instead.
     uint32_t wave, wave_coop, wave64;

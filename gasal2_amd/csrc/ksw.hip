@@ -28,10 +28,10 @@
 // less one gap open: with an end bonus no larger than that it never decides.
 //
 // Bound: packed VALU, 19 instructions per row pair and column (the dead diagonals
-// take two, the test four, the rank two), at 216 VGPRs and two waves per SIMD
-// (held to 168 for three, with 156 bytes spilled, the same 5.4 ms).  500,000
-// pairs of 100-250 bases: 26.2 -> 4.8 ms, 1,000 pairs 3.8 -> 1.3; 200,000
-// unrelated pairs, a fifth of them run again by k_ksw, 2.7 -> 1.5 ms.
+// take two, the test four, the rank two), at 228 VGPRs and two waves per SIMD
+// (held to 168 for three, with 156 bytes spilled, the same 5.4 ms).  DP of 500,000
+// pairs of 100-250 bases: 26.5 -> 4.5 ms, 1,000 pairs 3.7 -> 1.2; 200,000
+// unrelated pairs, a fifth of them run again by k_ksw, 2.4 -> 1.1 ms.
 #include "device.h"
 
 #include <type_traits>

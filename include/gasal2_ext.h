@@ -93,8 +93,9 @@ uint32_t gasal2_get_cigar(gasal_gpu_storage_t *s, uint32_t k, uint8_t *out, uint
  *     the lane path would spread over a fraction of the SIMDs (unless
  *     gasal2_set_wavefront or a tuned entry gives the thresholds); batches
  *     that the packed one-wave paths (4 to 256 lanes per pair) run faster
- *     than the lane kernels take those, WITH_TB while its checkpoints fit in
- *     the tile budget and in half of the free device memory;
+ *     than these take those, WITH_TB while its checkpoints fit in the tile
+ *     budget and in half of the free device memory and no sequence is empty
+ *     (one empty sequence keeps the whole batch off that path);
  *   1 reference-order kernels only (one lane per pair, no score tables);
  *   2 one lane per pair only (no one-wave-per-pair path);
  *   3 one wave per pair for every pair the path accepts (LOCAL without
