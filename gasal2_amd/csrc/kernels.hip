@@ -2583,7 +2583,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     uint4 q4 = {0u, 0u, 0u, 0u};   // recompute walks: cached query words
     uint32_t q4_key = 0xFFFFFFFFu;
     const int32_t nval = c.has_np ? -c.np : 0;
-    uint32_t ch[8];                 // cached 32-byte chunk: 8 columns of one 8x8 tile
+    uint32_t ch[8] = {0, 0, 0, 0, 0, 0, 0, 0};   // cached 32-byte chunk: 8 columns of one 8x8 tile
     int32_t ch_key = -1;
     uint32_t lut[8];                // score tables of the strip being recomputed (ck)
     int32_t lut_key = -1;
@@ -2606,7 +2606,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
     auto tile_key = [&](int32_t ii, int32_t jj) -> int32_t {
         const int32_t strip = (ii >> 3) + (jj >= read_len_8 ? 1 : 0);
         const int32_t col = jj >= read_len_8 ? jj - read_len_8 : jj;
-        return strip < TW ? strip * QW + (col >> 3) : -2;
+        return strip < TW && QW > 0 ? strip * QW + (col >> 3) : -2;   // an empty query has no tiles
     };
     bool done = !(i >= 0 && j >= 0);
     while (!done) {
@@ -2702,7 +2702,7 @@ __device__ __forceinline__ void tb_walk(const G2Dev &d, const G2Scores &c, uint3
             const int32_t strip = (i >> 3) + (j >= read_len_8 ? 1 : 0);
             const int32_t col = j >= read_len_8 ? j - read_len_8 : j;
             uint32_t cell_op = 0;
-            if (strip < TW) {
+            if (strip < TW && QW > 0) {
                 const int c7 = col & 7;
                 const uint32_t word = c7 < 4 ? (c7 < 2 ? (c7 == 0 ? ch[0] : ch[1]) : (c7 == 2 ? ch[2] : ch[3]))
                                              : (c7 < 6 ? (c7 == 4 ? ch[4] : ch[5]) : (c7 == 6 ? ch[6] : ch[7]));
