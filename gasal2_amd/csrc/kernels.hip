@@ -1806,7 +1806,7 @@ __device__ void lane_global_pk(const G2Dev &d, const G2Scores &c, const LaneCtx 
         if (__any(last_lo || last_hi)) words(std::true_type{});
         else words(std::false_type{});
     }
-    d.score[x.pair] = score;
+    d.score[x.pair] = C > 0 ? score : 0;   // no column: the step behind the last one was column 0
 }
 
 template <bool TB, bool LUT>
@@ -2094,6 +2094,10 @@ __global__ __launch_bounds__(64) void k_semi(G2Dev d, G2Scores c) {
     if (LUT && !TQ && d.pk16s) {   // packed 16-bit passes (values fit int16, tails on the target only)
         int32_t maxHH = MINUS_INF, maxY = read_len, sec = MINUS_INF, secy = read_len;
         semi_pass_pk<SECOND, HEAD, TT, false>(d, c, x, census, nval, 0, 0, maxHH, maxY, sec, secy);
+        // no column: the step behind the last one was column 0 (tested in the
+        // pass's loop, the compiler's registers for it ran a fourth wave a SIMD, and
+        // 300,000 pairs of 100-300 x 100-400 bases WITH_START 8.1 ms for 7.2)
+        if (QW == 0) { maxHH = sec = MINUS_INF; maxY = secy = read_len; }
         const uint32_t pr = x.pair;
         d.score[pr] = maxHH;
         d.tend[pr] = maxY;

@@ -48,3 +48,15 @@ def check(algo, start, second, tail, policy, scores=(1, 4, 6, 1)):
 def test_local_walk(second, policy, scores):
     """A pair without cells: the walk reads its first cell as 0, one match."""
     check(g.LOCAL, g.WITH_TB, second, g.TARGET, policy, scores)
+
+
+@pytest.mark.parametrize("policy", [0, 1, 2, 3])
+@pytest.mark.parametrize("algo,start,second", [(g.LOCAL, g.WITHOUT_START, False), (g.LOCAL, g.WITH_START, False),
+                                               (g.LOCAL, g.WITHOUT_START, True), (g.GLOBAL, g.WITHOUT_START, False),
+                                               (g.GLOBAL, g.WITH_TB, False), (g.SEMI_GLOBAL, g.WITHOUT_START, False),
+                                               (g.SEMI_GLOBAL, g.WITHOUT_START, True), (g.SEMI_GLOBAL, g.WITH_START, False),
+                                               (g.SEMI_GLOBAL, g.WITH_START, True), (g.BANDED, g.WITHOUT_START, False)])
+def test_scores(algo, start, second, policy):
+    """The packed lane kernels took the end of a query without columns from the strips' boundary."""
+    for tail in (g.NONE, g.TARGET, g.BOTH) if algo == g.SEMI_GLOBAL else (g.TARGET,):
+        check(algo, start, second, tail, policy)
