@@ -534,7 +534,7 @@ __global__ __launch_bounds__(256) void k_second_out(G2Dev d) {
 // read out of their lanes; a stretch of matches inside a tile is one step (the
 // first other cell on the diagonal, from the tile's 64-bit mask).  One lane per
 // pair (k_get_tb) waits for a tile's records and rebuilds it at every tile it
-// enters, 1.6 us per path cell: the walk of 64 pairs of 100-300 bases took 486 us
+// enters, 1.4 us per path cell: the walk of 64 pairs of 100-300 bases took 486 us
 // so, and takes 53; of 50,000 pairs of 50-5000 bases 8.7 ms, and takes 1.6.
 // Bound: of a lone pair the records' latency and a tile's recompute, once per 21
 // tiles of the diagonal; of many the two tiles in three rebuilt off the path.
